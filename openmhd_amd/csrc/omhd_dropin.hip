@@ -205,7 +205,7 @@ __global__ __launch_bounds__(256) void k_flux(double *__restrict__ F, const doub
     L[m] = VL[m * n + c];
     R[m] = VR[m * n + c];
   }
-  if (type == 3) hlld<D>(L, R, ch, ch * ch, f);
+  if (type == 3) hlld<D>(L, R, ch, ch * ch, f, moderate_pair(L, R));
   else riemann_other<D>(type, L, R, ch, ch * ch, f);
 #pragma unroll
   for (int m = 0; m < NV; m++) F[m * n + c] = f[m];

@@ -89,6 +89,13 @@ __device__ __forceinline__ void map_axis(int c, int n, int bc, unsigned slo, uns
   cm = cm < 0 ? 0 : (cm > n - 1 ? n - 1 : cm);  // lanes past the grid: any valid cell
 }
 
+// a wall's sign mask, hidden so that its nine sign bits are formed where a
+// wall is met and not held in scalar registers all along the march
+__device__ __forceinline__ unsigned here(unsigned mask) {
+  asm("" : "+s"(mask));
+  return mask;
+}
+
 // negate slot m when bit m of mask is set: a sign-bit XOR (exact, like the
 // reference's U(:,1,my) = -U(:,2,my))
 __device__ __forceinline__ double flip(double v, unsigned mask, int m) {
@@ -109,29 +116,29 @@ __device__ __forceinline__ void record_error(int *err, int code, int i, int j, i
 }
 
 // Per wavefront LDS: a ring of three primitive rows (rn-2, rn-1, rn) and the
-// carried left face state of the march-axis interface above row rn-2; for the
-// resistive flux also the transverse B samples of each ring row and Bx of the
-// row below the ring.  Keeping these out of VGPRs leaves ~18 live doubles
-// across each inlined HLLD call, so two wavefronts fit per SIMD.
+// carried left face state of the march-axis interface above row rn-2.
+// Keeping these out of VGPRs leaves ~18 live doubles across each inlined HLLD
+// call, so two wavefronts fit per SIMD.  Rows of exactly 64 entries (512 B):
+// the two-address LDS reads then reach every variable with immediate offsets.
+// 18432 B.
 struct SweepLds {
-  double ring[3][NV][66];  // [slot][var][lane + 1]; entries 0 and 65 repeat lanes 0 and 63
+  double ring[3][NV][64];  // [slot][var][lane]
   double wly[NV][64];
 };
 // The resistive passes keep the out-of-plane current terms of each row
 // already combined (same operations in the same order as the face formula,
 // so the same bits): xo the x-face term of each ring row, mo the march-axis
 // face term of the last two faces, prv the previous row's out-of-plane
-// samples.  XY pass: 22976 B (7 wavefronts per CU).
+// samples.  XY pass: 22528 B (7 wavefronts per CU).
 struct SweepLdsRes {
-  double ring[3][NV][66];
+  double ring[3][NV][64];
   double wly[NV][64];
   double xo[3][64];   // 0.25 (Bx(k+1)_c + Bx(k+1)_c+1 - Bx(k-1)_c - Bx(k-1)_c+1)
   double mo[2][64];   // 0.25 (By(k+1)_r-1 + By(k+1)_r - By(k-1)_r-1 - By(k-1)_r)
   double prv[2][64];  // By(k-1), By(k+1) of the previous row
-  double bxm[66];     // Bx of row rn-3
+  double bxm[64];     // Bx of row rn-3
 };
-// Z pass: no x-sweep, so the ring needs no halo entries (the Bz neighbours of
-// the z-face current come over DPP); 20480 B, 8 wavefronts per CU.
+// Z pass: 20480 B, 8 wavefronts per CU.
 struct SweepLdsResZ {
   double ring[3][NV][64];
   double wly[NV][64];
@@ -139,33 +146,252 @@ struct SweepLdsResZ {
   double prv[2][64];  // Bz(j-1), Bz(j+1) of the previous row
 };
 
-// Element of variable m at this lane's column of a row: `ro` is the row's
-// offset (uniform across the wavefront) and off8 the lane's byte offset in
-// the row.  The uniform part stays in scalar registers; the compiler adds the
-// lane's offset once per row and variable.
-__device__ __forceinline__ const double &lane_at(const double *a, long long plane, int m, long long ro,
-                                                 unsigned off8) {
+// The lane's element of a plane: a uniform base (scalar registers) plus the
+// lane's byte offset in the row, the form the scalar-base global instructions
+// take without address arithmetic in the vector unit.
+typedef __attribute__((address_space(1))) char gchar;
+typedef __attribute__((address_space(1))) double gdouble;
+// Walks the planes of a state at one row: `at` is the lane's element of the
+// current plane, `next` moves on.  The base is advanced by one scalar addition
+// per plane; hiding its value keeps the compiler from holding nine plane
+// addresses per state in (then spilled) scalar registers.
+struct PlaneWalk {
+  gchar *b;
+  long long step;
+  __device__ __forceinline__ PlaneWalk(const double *a, long long plane, long long ro)
+      : b((gchar *)(a + ro)), step(plane * 8) {
+    asm("" : "+s"(b));
+  }
+  __device__ __forceinline__ gdouble &at(unsigned off8) const { return *(gdouble *)(b + off8); }
+  __device__ __forceinline__ void next() {
+    b += step;
+    asm("" : "+s"(b));
+  }
+};
+template <int N>
+__device__ __forceinline__ void load_planes(const double *a, long long plane, long long ro, unsigned off8, double *v) {
+  PlaneWalk w(a, plane, ro);
+  asm("" : "+v"(off8));  // extended to 64 bits here, so that the loads take the 32-bit offset
+#pragma unroll
+  for (int m = 0; m < N; m++) {
+    v[m] = w.at(off8);
+    if (m + 1 < N) w.next();
+  }
+}
+__device__ __forceinline__ void store_planes(double *a, long long plane, long long ro, unsigned off8,
+                                             const double v[NV]) {
+  PlaneWalk w(a, plane, ro);
+  asm("" : "+v"(off8));
+#pragma unroll
+  for (int m = 0; m < NV; m++) {
+    w.at(off8) = v[m];
+    if (m + 1 < NV) w.next();
+  }
+}
+// one plane's element, for the few single reads
+__device__ __forceinline__ double lane_at(const double *a, long long plane, int m, long long ro, unsigned off8) {
   return *(const double *)((const char *)(a + (m * plane + ro)) + off8);
-}
-__device__ __forceinline__ double &lane_at(double *a, long long plane, int m, long long ro, unsigned off8) {
-  return *(double *)((char *)(a + (m * plane + ro)) + off8);
-}
-
-// Store this lane's value of a 66-entry LDS row: entry lane + 1, and again
-// at `edge`, the lane's second entry (0 for lane 0, 65 for lane 63, lane + 1
-// itself for the others).  Two plain stores per lane instead of lane tests
-// and divergent branches.
-__device__ __forceinline__ int edge66(int lane) { return lane == 0 ? 0 : (lane == 63 ? 65 : lane + 1); }
-__device__ __forceinline__ void put66(double *row, int lane, int edge, double v) {
-  row[lane + 1] = v;
-  row[edge] = v;
 }
 
 template <int RES, int PASS>
 using LdsOf = typename std::conditional<
     RES != 0, typename std::conditional<PASS == PASS_Z, SweepLdsResZ, SweepLdsRes>::type, SweepLds>::type;
 
+struct StepPar {
+  double ch, ch2, dtx, glm_f;
+};
+// the step's parameters; false: device dt mode halted by a stop (the state
+// stays as it was).  The block is written only between launches, so every
+// wavefront of a launch sees the same values.
+template <int STAGE>
+__device__ __forceinline__ bool step_par(const Sweep &p, StepPar &q) {
+  q = StepPar{p.ch, p.ch2, p.dtx, p.glm_f};
+  if (p.dpar) {
+    const DevPar *dp = (const DevPar *)p.dpar;
+    if (!(dp->dt > 0.0)) return false;
+    q = StepPar{dp->ch, dp->ch2, STAGE == 1 ? dp->dtx1 : dp->dtx2, dp->glm_f};
+  }
+  return true;
+}
+
+// One tile of a pass as a lane sees it: strip x chunk (x slice) of a grid.
+template <int PASS>
+struct TileView {
+  static constexpr int MD = PASS == PASS_Z ? 2 : 1;  // march axis = direction of its flux
+  static constexpr int ND = PASS == PASS_2D ? 2 : 3;
+  int c, cm, slice, nm, j0, hc;  // column, its mapped column, slice (k in XY, j in Z), march extent, chunk
+  long long rstride, fixoff;
+  unsigned xmask, cm8;           // the column's ghost signs, the lane's byte offset in a row
+  bool writer;
+  // lanes whose x-face (to the right) and march-axis face reach a written
+  // cell: the others' states may be far from their neighbours' and would only
+  // take the wavefront through more branches of the flux
+  bool xface, yface;
+  bool sane;  // no wall mirrors rho or p with a sign, so face states lie between their cells
+  __device__ __forceinline__ TileView(const Sweep &p, int t, int lane) {
+    const int strip = t % p.nstrip;
+    const int r2 = t / p.nstrip;
+    const int chunk = r2 % p.nchunk;
+    slice = r2 / p.nchunk;
+    c = strip * STRIP - 2 + lane;
+    nm = MD == 1 ? p.ny : p.nz;
+    j0 = chunk * p.rows;
+    hc = min(p.rows, nm - j0);
+    rstride = MD == 1 ? (long long)p.pitch : p.zstride;
+    fixoff = PASS == PASS_Z ? (long long)slice * p.pitch : (long long)slice * p.zstride;
+    map_axis(c, p.nx, p.bc[0], p.slo[0], p.shi[0], cm, xmask);
+    cm8 = (unsigned)cm * 8u;
+    writer = lane >= 2 && lane < 2 + STRIP && c < p.nx;
+    xface = lane >= 1 && lane < 2 + STRIP;
+    yface = lane >= 2 && lane < 2 + STRIP;
+    sane = ((p.slo[0] | p.shi[0] | p.slo[MD] | p.shi[MD]) & 0x18u) == 0u;
+  }
+  // offset of the first cell of (mapped) row rn, uniform across the wavefront
+  __device__ __forceinline__ long long row_off(const Sweep &p, int rn, unsigned &mask) const {
+    int rm;
+    unsigned ymask;
+    map_axis(rn, nm, p.bc[MD], p.slo[MD], p.shi[MD], rm, ymask);
+    mask = xmask ^ ymask;
+    return fixoff + (long long)rm * rstride;
+  }
+  // offset of an interior row (a writer lane's column c equals cm)
+  __device__ __forceinline__ long long own_off(int rn) const { return fixoff + (long long)rn * rstride; }
+
+  __device__ __forceinline__ void load_row(const Sweep &p, int rn, double u[NV], unsigned &mask) const {
+    load_planes<NV>(p.us, p.plane, row_off(p, rn, mask), cm8, u);
+  }
+  // ghost signs, glm_ss2 (main.f90:87), u2v and its positivity test on row rn;
+  // returns whether the row's cells are all moderate (cons_to_prim)
+  template <int STAGE>
+  __device__ __forceinline__ bool prim_row(const Sweep &p, double u[NV], unsigned mask, double glm_us, int rn,
+                                           double W[NV]) const {
+    if (any_lane(mask != 0u)) {  // a ghost row or column with negated slots (mirror faces)
+#pragma unroll
+      for (int m = 0; m < NV; m++) u[m] = flip(u[m], mask, m);
+    }
+    if constexpr (STAGE == 1) u[8] = glm_us * u[8];
+    const bool moderate = cons_to_prim(u, W);
+    if (!(W[3] > 0.0) || !(u[4] > 0.0)) {
+      int rm;
+      unsigned dummy;
+      map_axis(rn, nm, p.bc[MD], p.slo[MD], p.shi[MD], rm, dummy);
+      const int jj = MD == 1 ? rm : slice;
+      const int kk = MD == 1 ? (ND == 3 ? slice + 2 : 0) : rm + 2;
+      record_error(p.err, ((W[3] > 0.0) ? OMHD_ERR_DENSITY : OMHD_ERR_PRESSURE) | (STAGE == 2 ? ERR_IN_USTAR : 0),
+                   cm + 2, jj + 2, kk);
+    }
+    return moderate;
+  }
+  // the mirror of an x wall face
+  __device__ __forceinline__ void x_wall(const Sweep &p, double L[NV], double R[NV]) const {
+    if (p.bc[0] == OMHD_BC_MIRROR) {
+      if (c == -1) {
+        const unsigned sg = here(p.slo[0]);
+#pragma unroll
+        for (int m = 0; m < NV; m++) L[m] = flip(R[m], sg, m);
+      }
+      if (c == p.nx - 1) {
+        const unsigned sg = here(p.shi[0]);
+#pragma unroll
+        for (int m = 0; m < NV; m++) R[m] = flip(L[m], sg, m);
+      }
+    }
+  }
+  // the mirror of a march-axis wall face: bc_for_G, 2D_KH/bc.f90:62-81
+  __device__ __forceinline__ void march_wall(const Sweep &p, int upper, double L[NV], double R[NV]) const {
+    if (p.bc[MD] == OMHD_BC_MIRROR) {
+      if (upper == 0) {
+        const unsigned sg = here(p.slo[MD]);
+#pragma unroll
+        for (int m = 0; m < NV; m++) L[m] = flip(R[m], sg, m);
+      }
+      if (upper == nm) {
+        const unsigned sg = here(p.shi[MD]);
+#pragma unroll
+        for (int m = 0; m < NV; m++) R[m] = flip(L[m], sg, m);
+      }
+    }
+  }
+};
+
+// Next step's u2v and set_dt on a cell of U^{n+1}
+template <int ND>
+__device__ __forceinline__ void next_speed(const Sweep &p, const double o9[NV], double &vloc) {
+  double w2[NV];
+  const bool moderate = cons_to_prim(o9, w2);
+  if (!(w2[3] > 0.0) || !(o9[4] > 0.0))
+    (void)atomicCAS(p.err_next, 0, (w2[3] > 0.0) ? OMHD_ERR_DENSITY : OMHD_ERR_PRESSURE);
+  const double vt = cell_speed<ND>(o9, w2, moderate);
+  vloc = (vt > vloc || !(vt == vt)) ? vt : vloc;
+}
+__device__ __forceinline__ void reduce_speed(const Sweep &p, double vloc, int lane) {
+  if (!(vloc >= 0.0)) (void)atomicCAS(p.err_next + 1, 0, OMHD_ERR_DT);
+  const double vm = wave_max(vloc >= 0.0 ? vloc : 0.0);
+  if (lane == 0) atomic_max_nonneg(p.vmax_bits, vm);
+}
+
+// out-of-plane samples of the resistive XY pass: Bx (0, 1) and By (2, 3) of
+// row r in planes k-1 and k+1, as loaded and, after `signed_aux`, with the
+// ghost signs
+template <int PASS>
+__device__ __forceinline__ void aux_load(const Sweep &p, const TileView<PASS> &v, int r, double a[4]) {
+  int rm;
+  unsigned ym;
+  map_axis(r, v.nm, p.bc[1], p.slo[1], p.shi[1], rm, ym);
+#pragma unroll
+  for (int s2 = 0; s2 < 2; s2++) {
+    int km;
+    unsigned zm;
+    map_axis(v.slice + (s2 ? 1 : -1), p.nz, p.bc[2], p.slo[2], p.shi[2], km, zm);
+    const long long ro = (long long)km * p.zstride + (long long)rm * p.pitch;
+    a[s2] = lane_at(p.us, p.plane, 5, ro, v.cm8);
+    a[2 + s2] = lane_at(p.us, p.plane, 6, ro, v.cm8);
+  }
+}
+template <int PASS>
+__device__ __forceinline__ void signed_aux(const Sweep &p, const TileView<PASS> &v, unsigned mask, double a[4]) {
+#pragma unroll
+  for (int s2 = 0; s2 < 2; s2++) {
+    int km;
+    unsigned zm;
+    map_axis(v.slice + (s2 ? 1 : -1), p.nz, p.bc[2], p.slo[2], p.shi[2], km, zm);
+    a[s2] = flip(a[s2], mask ^ zm, 5);
+    a[2 + s2] = flip(a[2 + s2], mask ^ zm, 6);
+  }
+}
+// out-of-plane samples of the resistive Z pass: Bz of row r in slices j-1 (0)
+// and j+1 (1), ghost signs applied
+template <int PASS>
+__device__ __forceinline__ void z_samples(const Sweep &p, const TileView<PASS> &v, int r, unsigned mask, double bz[2]) {
+  int rm;
+  unsigned zmask;
+  map_axis(r, v.nm, p.bc[2], p.slo[2], p.shi[2], rm, zmask);
+#pragma unroll
+  for (int s2 = 0; s2 < 2; s2++) {
+    int jm;
+    unsigned jmask;
+    map_axis(v.slice + (s2 ? 1 : -1), p.ny, p.bc[1], p.slo[1], p.shi[1], jm, jmask);
+    const long long ro = (long long)rm * p.zstride + (long long)jm * p.pitch;
+    bz[s2] = flip(lane_at(p.us, p.plane, 7, ro, v.cm8), mask ^ jmask, 7);
+  }
+}
+// x-face (c+1/2) term of a row: flux_resistive.cuf:89-91's k-differences of Bx
+__device__ __forceinline__ double xo_term(const double a[4]) {
+  return 0.25 * (a[1] + from_next(a[1]) - a[0] - from_next(a[0]));
+}
+
 // One tile: strip x chunk (x slice) of one grid.
+// The XY and 2D passes are bound by the vector unit's issue slots and by what
+// of a row's serial chain two wavefronts per SIMD leave uncovered; the Z pass
+// by HBM.  On KH 4096^2 (minmod) a row takes 1301 vector instructions in stage
+// 1 and 1453 in stage 2, two thirds of them the two flux evaluations, and the
+// vector unit issues in 80% and 75% of the cycles: 0.89 and 1.03 ms a stage.
+// With a division for every quotient, 64-bit address arithmetic per access and
+// wall signs held in (spilled) scalar registers it was 1516 and 1687
+// instructions, 86% and 83% busy, 0.99 and 1.12 ms.  So what is not arithmetic
+// of the scheme is kept out of the vector unit: scalar bases for loads and
+// stores, wall signs formed only at walls, ring rows of 512 B, the lane masks
+// of compares used as they are.
 // PREF: stage 2 issues the U^n loads of the combined row early (where the
 // register budget allows it without spills: the resident kernels, not the
 // ensemble kernel, whose per-member parameters take more registers).
@@ -174,85 +400,66 @@ template <int LIM, int STAGE, int TT, int PASS, int RES, bool PREF = true, bool 
 __device__ __forceinline__ void march_tile(const Sweep &p, const int t, LdsOf<RES, PASS> &lds) {
   constexpr bool XS = PASS != PASS_Z;         // x-sweep of the oldest row
   constexpr bool FINAL = PASS != PASS_XY;     // RK update (else write acc)
-  constexpr int MD = PASS == PASS_Z ? 2 : 1;  // march axis = direction of its HLLD
-  constexpr int ND = PASS == PASS_2D ? 2 : 3;
+  constexpr int MD = TileView<PASS>::MD, ND = TileView<PASS>::ND;
   const int lane = threadIdx.x;
-  const int edge = edge66(lane);
-  constexpr int RO = (RES != 0 && PASS == PASS_Z) ? 0 : 1;  // first own entry of a ring row
-  const int strip = t % p.nstrip;
-  const int r2 = t / p.nstrip;
-  const int chunk = r2 % p.nchunk, slice = r2 / p.nchunk;  // slice: k (XY) or j (Z)
-  const int c = strip * STRIP - 2 + lane;
-  const int nm = MD == 1 ? p.ny : p.nz;  // cells along the march axis
-  const int j0 = chunk * p.rows;
-  const int hc = min(p.rows, nm - j0);
-  const long long rstride = MD == 1 ? (long long)p.pitch : p.zstride;
-  const long long fixoff = PASS == PASS_Z ? (long long)slice * p.pitch : (long long)slice * p.zstride;
-  int cm;
-  unsigned xmask;
-  map_axis(c, p.nx, p.bc[0], p.slo[0], p.shi[0], cm, xmask);
-  const bool writer = lane >= 2 && lane < 2 + STRIP && c < p.nx;
-  const bool xlo_face = p.bc[0] == OMHD_BC_MIRROR && c == -1;
-  const bool xhi_face = p.bc[0] == OMHD_BC_MIRROR && c == p.nx - 1;
-  double ch = p.ch, ch2 = p.ch2, dtx = p.dtx, glm_f = p.glm_f;
-  if (p.dpar) {
-    const DevPar *dp = (const DevPar *)p.dpar;
-    if (!(dp->dt > 0.0)) return;  // device dt mode halted by a stop: the state stays as it was
-    ch = dp->ch;
-    ch2 = dp->ch2;
-    dtx = STAGE == 1 ? dp->dtx1 : dp->dtx2;
-    glm_f = dp->glm_f;
-  }
-  const double glm_us = (STAGE == 1) ? glm_f : 1.0;
-  const long long plane = p.plane;
+  const int lm = (lane + 63) & 63, lp = (lane + 1) & 63;  // the edge lanes' flux reaches no written cell
   const int ix = p.nx + 2, jx = p.ny + 2;
-
+  StepPar q;
+  if (!step_par<STAGE>(p, q)) return;
+  const TileView<PASS> v(p, t, lane);
+  const double glm_us = (STAGE == 1) ? q.glm_f : 1.0;
   double Gl[NV], nxt[NV];
   double vloc = 0.0;
-
-  const unsigned cm8 = (unsigned)cm * 8u;  // this lane's byte offset in a row
-  // offset of the first cell of (mapped) row rn, uniform across the wavefront
-  auto row_off = [&](int rn, unsigned &mask) -> long long {
-    int rm;
-    unsigned ymask;
-    map_axis(rn, nm, p.bc[MD], p.slo[MD], p.shi[MD], rm, ymask);
-    mask = xmask ^ ymask;
-    return fixoff + (long long)rm * rstride;
-  };
-
+  bool okA = false, okB = false, okC = false;  // rows rn-2, rn-1, rn: every cell moderate
   unsigned mask_nxt;
-  {
-    const long long ro = row_off(j0 - 2, mask_nxt);
-#pragma unroll
-    for (int m = 0; m < NV; m++) nxt[m] = lane_at(p.us, plane, m, ro, cm8);
-  }
-  // resistive XY pass: Bx and By of row r in planes k-1 and k+1 (as loaded,
-  // before the ghost signs), prefetched one row ahead like the row itself
-  auto aux_load = [&](int r, double a[4]) {
-    int rm;
-    unsigned ym;
-    map_axis(r, nm, p.bc[MD], p.slo[MD], p.shi[MD], rm, ym);
-#pragma unroll
-    for (int s2 = 0; s2 < 2; s2++) {
-      int km;
-      unsigned zm;
-      map_axis(slice + (s2 ? 1 : -1), p.nz, p.bc[2], p.slo[2], p.shi[2], km, zm);
-      const long long ro = (long long)km * p.zstride + (long long)rm * p.pitch;
-      a[s2] = lane_at(p.us, plane, 5, ro, cm8);
-      a[2 + s2] = lane_at(p.us, plane, 6, ro, cm8);
-    }
-  };
+  // resistive XY pass: Bx and By of the next row in planes k-1 and k+1,
+  // prefetched one row ahead like the row itself
   double auxn[4] = {0.0, 0.0, 0.0, 0.0};
-  if constexpr (RES != 0 && PASS == PASS_XY) aux_load(j0 - 2, auxn);
-
   // resistive Z pass: the z-face eta/dx of this lane's column and the tile's
   // slice, the same for every row of the march
   double etz_dx = 0.0;
   if constexpr (RES != 0 && PASS == PASS_Z)
-    etz_dx = p.eta[2 * (size_t)ix * jx + (size_t)(cm + 1) + (size_t)ix * (slice + 1)] / p.dx;
-  for (int k = 0; k < hc + 4; ++k) {
-    const int rn = j0 - 2 + k;
-    const int sa = (k + 1) % 3, sb = (k + 2) % 3, sc = k % 3;  // rows rn-2, rn-1, rn
+    etz_dx = p.eta[2 * (size_t)ix * jx + (size_t)(v.cm + 1) + (size_t)ix * (v.slice + 1)] / p.dx;
+  // the first two rows, loaded together with the third: one memory latency
+  // before the march instead of three
+  {
+    double u[2][NV], a[2][4];
+    unsigned mk[2];
+#pragma unroll
+    for (int r = 0; r < 2; r++) {
+      v.load_row(p, v.j0 - 2 + r, u[r], mk[r]);
+      if constexpr (RES != 0 && PASS == PASS_XY) aux_load(p, v, v.j0 - 2 + r, a[r]);
+    }
+    v.load_row(p, v.j0, nxt, mask_nxt);
+    if constexpr (RES != 0 && PASS == PASS_XY) aux_load(p, v, v.j0, auxn);
+#pragma unroll
+    for (int r = 0; r < 2; r++) {
+      double W[NV];
+      okB = okC;
+      okC = v.template prim_row<STAGE>(p, u[r], mk[r], glm_us, v.j0 - 2 + r, W);
+#pragma unroll
+      for (int m = 0; m < NV; m++) lds.ring[r][m][lane] = W[m];
+      if constexpr (RES != 0 && PASS == PASS_XY) {
+        signed_aux(p, v, mk[r], a[r]);
+        lds.xo[r][lane] = xo_term(a[r]);
+        lds.prv[0][lane] = a[r][2];
+        lds.prv[1][lane] = a[r][3];
+      }
+      if constexpr (RES != 0 && PASS == PASS_Z) {
+        double bz[2];
+        z_samples(p, v, v.j0 - 2 + r, mk[r], bz);
+        lds.prv[0][lane] = bz[0];
+        lds.prv[1][lane] = bz[1];
+      }
+    }
+  }
+  int sa = 2, sb = 0, sc = 1;  // ring slots of rows rn-2, rn-1, rn
+  for (int k = 2; k < v.hc + 4; ++k) {
+    const int rn = v.j0 - 2 + k;
+    const int s0 = sa;
+    sa = sb;
+    sb = sc;
+    sc = s0;
     // resistive XY pass: this iteration's x- and y-face eta/dx, loaded here so
     // that their latency hides behind the row's work.  The row index is
     // clamped into the table (the warm-up iterations do not use the values),
@@ -260,115 +467,62 @@ __device__ __forceinline__ void march_tile(const Sweep &p, const int t, LdsOf<RE
     double etx_dx = 0.0, ety_dx = 0.0;
     if constexpr (RES != 0 && PASS == PASS_XY) {
       const int re = min(max(rn - 1, 0), jx - 1);
-      const int cf = min(max(c + 1, 0), ix - 1);
+      const int cf = min(max(v.c + 1, 0), ix - 1);
       etx_dx = p.eta[(size_t)cf + (size_t)ix * re] / p.dx;
-      ety_dx = p.eta[(size_t)ix * jx + (size_t)(cm + 1) + (size_t)ix * re] / p.dx;
+      ety_dx = p.eta[(size_t)ix * jx + (size_t)(v.cm + 1) + (size_t)ix * re] / p.dx;
     }
     {
-      double u[NV], W[NV];
-      if (__any(mask_nxt != 0u)) {  // a ghost row or column with negated slots (mirror faces)
+      double W[NV], aux[4];
+      const unsigned mask = mask_nxt;
+      okA = okB;
+      okB = okC;
+      okC = v.template prim_row<STAGE>(p, nxt, mask, glm_us, rn, W);
 #pragma unroll
-        for (int m = 0; m < NV; m++) u[m] = flip(nxt[m], mask_nxt, m);
-      } else {
-#pragma unroll
-        for (int m = 0; m < NV; m++) u[m] = nxt[m];
+      for (int e = 0; e < 4; e++) aux[e] = auxn[e];
+      if (k + 1 < v.hc + 4) {  // prefetch the next row
+        v.load_row(p, rn + 1, nxt, mask_nxt);
+        if constexpr (RES != 0 && PASS == PASS_XY) aux_load(p, v, rn + 1, auxn);
       }
-      u[8] = glm_us * u[8];  // glm_ss2 before the sweep (main.f90:87)
-      double auxc[4];
-#pragma unroll
-      for (int q = 0; q < 4; q++) auxc[q] = auxn[q];
       if constexpr (RES != 0 && PASS == PASS_XY) {
-        if (k + 1 < hc + 4) aux_load(rn + 1, auxn);
-      }
-      if (k + 1 < hc + 4) {  // prefetch the next row
-        unsigned mnext;
-        const long long ro = row_off(rn + 1, mnext);
-#pragma unroll
-        for (int m = 0; m < NV; m++) nxt[m] = lane_at(p.us, plane, m, ro, cm8);
-        mask_nxt = mnext;
-      }
-      cons_to_prim(u, W);  // u2v
-      if (!(W[3] > 0.0) || !(u[4] > 0.0)) {
-        int rm;
-        unsigned dummy;
-        map_axis(rn, nm, p.bc[MD], p.slo[MD], p.shi[MD], rm, dummy);
-        const int jj = MD == 1 ? rm : slice;
-        const int kk = MD == 1 ? (ND == 3 ? slice + 2 : 0) : rm + 2;
-        record_error(p.err, ((W[3] > 0.0) ? OMHD_ERR_DENSITY : OMHD_ERR_PRESSURE) | (STAGE == 2 ? ERR_IN_USTAR : 0),
-                     cm + 2, jj + 2, kk);
-      }
-      if constexpr (RES != 0) {
         // transverse B samples of this row for the resistive face currents
-        int rm;
-        unsigned ymask;
-        map_axis(rn, nm, p.bc[MD], p.slo[MD], p.shi[MD], rm, ymask);
-        if constexpr (PASS == PASS_XY) {
-          put66(lds.bxm, lane, edge, lds.ring[sc][5][lane + 1]);  // Bx of row rn-3, before its slot is reused
-          double bx[2], by[2];  // planes k-1 (0) and k+1 (1), ghost signs applied
-#pragma unroll
-          for (int s2 = 0; s2 < 2; s2++) {
-            int km;
-            unsigned zmask;
-            map_axis(slice + (s2 ? 1 : -1), p.nz, p.bc[2], p.slo[2], p.shi[2], km, zmask);
-            const unsigned mk = xmask ^ ymask ^ zmask;
-            bx[s2] = flip(auxc[s2], mk, 5);
-            by[s2] = flip(auxc[2 + s2], mk, 6);
-          }
-          // x-face (c+1/2) term of row rn: flux_resistive.cuf:89-91's k-differences of Bx
-          lds.xo[sc][lane] = 0.25 * (bx[1] + from_next(bx[1]) - bx[0] - from_next(bx[0]));
-          // y-face (rn-1/2) term: flux_resistive.cuf:106-108's k-differences of By
-          lds.mo[k & 1][lane] = 0.25 * (lds.prv[1][lane] + by[1] - lds.prv[0][lane] - by[0]);
-          lds.prv[0][lane] = by[0];
-          lds.prv[1][lane] = by[1];
-        } else {
-          double bz[2];  // slices j-1 (0) and j+1 (1), ghost signs applied
-#pragma unroll
-          for (int s2 = 0; s2 < 2; s2++) {
-            int jm;
-            unsigned jmask;
-            map_axis(slice + (s2 ? 1 : -1), p.ny, p.bc[1], p.slo[1], p.shi[1], jm, jmask);
-            const unsigned mk = xmask ^ ymask ^ jmask;
-            const long long ro = (long long)rm * p.zstride + (long long)jm * p.pitch;
-            bz[s2] = flip(lane_at(p.us, plane, 7, ro, cm8), mk, 7);
-          }
-          // z-face (rn-1/2) term: flux_resistive.cuf:123-125's j-differences of Bz
-          lds.mo[k & 1][lane] = 0.25 * (lds.prv[1][lane] + bz[1] - lds.prv[0][lane] - bz[0]);
-          lds.prv[0][lane] = bz[0];
-          lds.prv[1][lane] = bz[1];
-        }
+        lds.bxm[lane] = lds.ring[sc][5][lane];  // Bx of row rn-3, before its slot is reused
+        signed_aux(p, v, mask, aux);
+        lds.xo[sc][lane] = xo_term(aux);
+        // y-face (rn-1/2) term: flux_resistive.cuf:106-108's k-differences of By
+        lds.mo[k & 1][lane] = 0.25 * (lds.prv[1][lane] + aux[3] - lds.prv[0][lane] - aux[2]);
+        lds.prv[0][lane] = aux[2];
+        lds.prv[1][lane] = aux[3];
+      }
+      if constexpr (RES != 0 && PASS == PASS_Z) {
+        double bz[2];
+        z_samples(p, v, rn, mask, bz);
+        // z-face (rn-1/2) term: flux_resistive.cuf:123-125's j-differences of Bz
+        lds.mo[k & 1][lane] = 0.25 * (lds.prv[1][lane] + bz[1] - lds.prv[0][lane] - bz[0]);
+        lds.prv[0][lane] = bz[0];
+        lds.prv[1][lane] = bz[1];
       }
 #pragma unroll
-      for (int m = 0; m < NV; m++) {
-        if constexpr (RO == 0) lds.ring[sc][m][lane] = W[m];
-        else put66(lds.ring[sc][m], lane, edge, W[m]);
-      }
+      for (int m = 0; m < NV; m++) lds.ring[sc][m][lane] = W[m];
     }
     __syncthreads();  // one wavefront per workgroup: orders the ring writes before the neighbour reads
-    // stage 2: issue the loads of U^n for the row combined at the end of this
-    // iteration now, so their latency hides behind the two flux evaluations
+    // the update's own-cell loads go out now, so their latency hides behind
+    // the flux evaluations.  TVD stage 2 folds U^n + U* (the first sum of
+    // rk_tvd22) before the march-axis flux, so the U* loads go out as one batch
     double a0p[NV], usp[NV];
-    // TVD stage 2 folds U^n + U* (the first sum of rk_tvd22) before the
-    // march-axis flux, so the U* loads go out as one batch
     constexpr bool FOLD = FINAL && STAGE == 2 && TT == 0 && PREF;
-    // row rn-2, combined in this iteration: its offset (a writer lane's column c equals cm)
-    const long long ro2 = fixoff + (long long)(rn - 2) * rstride;
+    const long long ro2 = v.own_off(rn - 2);  // row rn-2, updated in this iteration
     if constexpr (FINAL && STAGE == 2 && PREF) {
-      if (k >= 4 && writer) {
-#pragma unroll
-        for (int m = 0; m < NV; m++) a0p[m] = lane_at(p.u0, plane, m, ro2, cm8);
-      }
+      if (k >= 4 && v.writer) load_planes<NV>(p.u0, p.plane, ro2, v.cm8, a0p);
     }
     if constexpr (FINAL && STAGE == 1 && PREF) {
-      if (k >= 4 && writer) {
+      if (k >= 4 && v.writer) {
+        // slots 4-8 (rho, B, psi) of a primitive row are the conserved ones
+        // (psi with the glm factor of stage 1 applied), and the row updated
+        // here is an interior row of the LDS ring: only slots 0-3 are read
+        // again from memory
+        load_planes<4>(p.us, p.plane, ro2, v.cm8, usp);
 #pragma unroll
-        for (int m = 0; m < NV; m++) {
-          // slots 4-8 (rho, B, psi) of a primitive row are the conserved
-          // ones (psi with the glm factor of stage 1 applied), and the row
-          // combined here is an interior row of the LDS ring: only slots
-          // 0-3 are read again from memory
-          if (m < 4) usp[m] = lane_at(p.us, plane, m, ro2, cm8);
-          else usp[m] = lds.ring[sa][m][lane + RO];
-        }
+        for (int m = 4; m < NV; m++) usp[m] = lds.ring[sa][m][lane];
       }
     }
     // Z pass, stage 1, ideal MHD: the XY pass's partial flux difference for
@@ -376,10 +530,7 @@ __device__ __forceinline__ void march_tile(const Sweep &p, const int t, LdsOf<RE
     constexpr bool ZPRE = PASS == PASS_Z && PREF && RES == 0 && STAGE == 1;
     double azp[NV];
     if constexpr (ZPRE) {
-      if (k >= 4 && writer) {
-#pragma unroll
-        for (int m = 0; m < NV; m++) azp[m] = lane_at((const double *)p.acc, plane, m, ro2, cm8);
-      }
+      if (k >= 4 && v.writer) load_planes<NV>(p.acc, p.plane, ro2, v.cm8, azp);
     }
 
     // x-sweep of row r = rn-2: tq = (F(i-1) - F(i)) + G(j-1)   (rk.f90:30-31 order)
@@ -388,15 +539,15 @@ __device__ __forceinline__ void march_tile(const Sweep &p, const int t, LdsOf<RE
       if (k >= 4) {
         double Lx[NV], Rx[NV], F[NV];
         {
-          // all 27 neighbour reads in flight before the first slope: left to
-          // itself the scheduler issues them three at a time and waits on each
-          // group (one LDS latency per variable)
+          // all neighbour reads in flight before the first slope: left to
+          // itself the scheduler issues them three at a time and waits on
+          // each group (one LDS latency per variable)
           double x0[NV], x1[NV], x2[NV];
 #pragma unroll
           for (int m = 0; m < NV; m++) {
-            x0[m] = lds.ring[sa][m][lane];
-            x1[m] = lds.ring[sa][m][lane + 1];
-            x2[m] = lds.ring[sa][m][lane + 2];
+            x0[m] = lds.ring[sa][m][lm];
+            x1[m] = lds.ring[sa][m][lane];
+            x2[m] = lds.ring[sa][m][lp];
           }
           __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -406,33 +557,26 @@ __device__ __forceinline__ void march_tile(const Sweep &p, const int t, LdsOf<RE
             Rx[m] = from_next(wRx);
           }
         }
-        if (xlo_face) {
-#pragma unroll
-          for (int m = 0; m < NV; m++) Lx[m] = flip(Rx[m], p.slo[0], m);
+        v.x_wall(p, Lx, Rx);
+        if (v.xface) {
+          if constexpr (GEN) riemann_other<0>(p.ftype, Lx, Rx, q.ch, q.ch2, F);
+          else hlld<0>(Lx, Rx, q.ch, q.ch2, F, v.sane && okA);
         }
-        if (xhi_face) {
-#pragma unroll
-          for (int m = 0; m < NV; m++) Rx[m] = flip(Lx[m], p.shi[0], m);
-        }
-        if constexpr (GEN) riemann_other<0>(p.ftype, Lx, Rx, ch, ch2, F);
-        else hlld<0>(Lx, Rx, ch, ch2, F);
         if constexpr (RES != 0) {  // flux_resistive.cuf:89-101 at x-face (c+1/2, row rn-2, plane slice)
-          const int l = lane + 1;
           const double *A6 = lds.ring[sa][6], *A7 = lds.ring[sa][7];
           const double *B5 = lds.ring[sb][5];
-          const double JyS = -(A7[l + 1] - A7[l]) + lds.xo[sa][lane];
-          const double JzS = (A6[l + 1] - A6[l]) - 0.25 * (B5[l] + B5[l + 1] - lds.bxm[l] - lds.bxm[l + 1]);
-          const double eta_dx = etx_dx;
-          F[3] = F[3] + 0.5 * eta_dx * (JyS * (A7[l] + A7[l + 1]) - JzS * (A6[l] + A6[l + 1]));
-          F[6] = F[6] - eta_dx * JzS;
-          F[7] = F[7] + eta_dx * JyS;
+          const double JyS = -(A7[lp] - A7[lane]) + lds.xo[sa][lane];
+          const double JzS = (A6[lp] - A6[lane]) - 0.25 * (B5[lane] + B5[lp] - lds.bxm[lane] - lds.bxm[lp]);
+          F[3] = F[3] + 0.5 * etx_dx * (JyS * (A7[lane] + A7[lp]) - JzS * (A6[lane] + A6[lp]));
+          F[6] = F[6] - etx_dx * JzS;
+          F[7] = F[7] + etx_dx * JyS;
         }
 #pragma unroll
         for (int m = 0; m < NV; m++) tq[m] = from_prev(F[m]) - F[m] + Gl[m];
       }
     }
 
-    if (k >= 2) {
+    {
       // march-axis slopes of row rn-1 from rows rn-2, rn-1, rn
       double Lf[NV], Rf[NV];
       double y0[NV];  // row rn-2 as the ring holds it (also stage 2's fold below)
@@ -440,9 +584,9 @@ __device__ __forceinline__ void march_tile(const Sweep &p, const int t, LdsOf<RE
         double y1[NV], y2[NV];  // likewise: every own-lane read before the first slope
 #pragma unroll
         for (int m = 0; m < NV; m++) {
-          y0[m] = lds.ring[sa][m][lane + RO];
-          y1[m] = lds.ring[sb][m][lane + RO];
-          y2[m] = lds.ring[sc][m][lane + RO];
+          y0[m] = lds.ring[sa][m][lane];
+          y1[m] = lds.ring[sb][m][lane];
+          y2[m] = lds.ring[sc][m][lane];
           Lf[m] = lds.wly[m][lane];  // left state of the interface above row rn-2
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -454,113 +598,86 @@ __device__ __forceinline__ void march_tile(const Sweep &p, const int t, LdsOf<RE
         }
       }
       if constexpr (FOLD) {
-        if (k >= 4 && writer) {
+        if (k >= 4 && v.writer) {
           double usf[NV];  // U* of row rn-2: slots 4-8 as the ring holds them (y0)
+          load_planes<4>(p.us, p.plane, ro2, v.cm8, usf);
 #pragma unroll
-          for (int m = 0; m < NV; m++) usf[m] = m < 4 ? lane_at(p.us, plane, m, ro2, cm8) : y0[m];
+          for (int m = 4; m < NV; m++) usf[m] = y0[m];
 #pragma unroll
-          for (int m = 0; m < NV; m++) a0p[m] = (m == 8 ? glm_f * a0p[m] : a0p[m]) + usf[m];
+          for (int m = 0; m < NV; m++) a0p[m] = (m == 8 ? q.glm_f * a0p[m] : a0p[m]) + usf[m];
         }
       }
       if (k >= 3) {
-        // march-axis interface between rows rn-2 and rn-1
-        if (p.bc[MD] == OMHD_BC_MIRROR) {
-          if (rn - 1 == 0) {  // low wall: bc_for_G, 2D_KH/bc.f90:62-70
-#pragma unroll
-            for (int m = 0; m < NV; m++) Lf[m] = flip(Rf[m], p.slo[MD], m);
-          }
-          if (rn - 1 == nm) {  // high wall: 2D_KH/bc.f90:73-81
-#pragma unroll
-            for (int m = 0; m < NV; m++) Rf[m] = flip(Lf[m], p.shi[MD], m);
-          }
-        }
+        v.march_wall(p, rn - 1, Lf, Rf);  // the interface between rows rn-2 and rn-1
         double G[NV];
-        if constexpr (GEN) riemann_other<MD>(p.ftype, Lf, Rf, ch, ch2, G);
-        else hlld<MD>(Lf, Rf, ch, ch2, G);
+        if (v.yface) {
+          if constexpr (GEN) riemann_other<MD>(p.ftype, Lf, Rf, q.ch, q.ch2, G);
+          else hlld<MD>(Lf, Rf, q.ch, q.ch2, G, v.sane && okA && okB);
+        }
         if constexpr (RES != 0) {
-          const int l = lane + RO;
           const double *A5 = lds.ring[sa][5], *A6 = lds.ring[sa][6], *A7 = lds.ring[sa][7];
           const double *B5 = lds.ring[sb][5], *B6 = lds.ring[sb][6], *B7 = lds.ring[sb][7];
           if constexpr (PASS == PASS_XY) {  // flux_resistive.cuf:106-118, y-face (c, rn-2 + 1/2, slice)
-            const double JxS = (B7[l] - A7[l]) - lds.mo[(k + 1) & 1][lane];
-            const double JzS = -(B5[l] - A5[l]) + 0.25 * (A6[l + 1] + B6[l + 1] - A6[l - 1] - B6[l - 1]);
-            const double eta_dx = ety_dx;
-            G[3] = G[3] + 0.5 * eta_dx * (JzS * (A5[l] + B5[l]) - JxS * (A7[l] + B7[l]));
-            G[5] = G[5] + eta_dx * JzS;
-            G[7] = G[7] - eta_dx * JxS;
+            const double JxS = (B7[lane] - A7[lane]) - lds.mo[(k + 1) & 1][lane];
+            const double JzS = -(B5[lane] - A5[lane]) + 0.25 * (A6[lp] + B6[lp] - A6[lm] - B6[lm]);
+            G[3] = G[3] + 0.5 * ety_dx * (JzS * (A5[lane] + B5[lane]) - JxS * (A7[lane] + B7[lane]));
+            G[5] = G[5] + ety_dx * JzS;
+            G[7] = G[7] - ety_dx * JxS;
           } else {  // flux_resistive.cuf:123-135, z-face (c, slice, rn-2 + 1/2)
-            const double a7 = A7[l], b7 = B7[l];  // column neighbours over DPP (the edge lanes write nothing)
-            const double JyS = (B5[l] - A5[l]) - 0.25 * (from_next(a7) + from_next(b7) - from_prev(a7) - from_prev(b7));
-            const double JxS = -(B6[l] - A6[l]) + lds.mo[(k + 1) & 1][lane];
-            const double eta_dx = etz_dx;
-            G[3] = G[3] + 0.5 * eta_dx * (JxS * (A6[l] + B6[l]) - JyS * (A5[l] + B5[l]));
-            G[5] = G[5] - eta_dx * JyS;
-            G[6] = G[6] + eta_dx * JxS;
+            const double JyS = (B5[lane] - A5[lane]) - 0.25 * (A7[lp] + B7[lp] - A7[lm] - B7[lm]);
+            const double JxS = -(B6[lane] - A6[lane]) + lds.mo[(k + 1) & 1][lane];
+            G[3] = G[3] + 0.5 * etz_dx * (JxS * (A6[lane] + B6[lane]) - JyS * (A5[lane] + B5[lane]));
+            G[5] = G[5] - etz_dx * JyS;
+            G[6] = G[6] + etz_dx * JxS;
           }
         }
 
-        if (k >= 4 && writer) {
+        if (k >= 4 && v.writer) {
           double d[NV];
           if constexpr (PASS == PASS_2D) {
 #pragma unroll
             for (int m = 0; m < NV; m++) d[m] = tq[m] - G[m];
           } else if constexpr (PASS == PASS_XY) {
 #pragma unroll
-            for (int m = 0; m < NV; m++) lane_at(p.acc, plane, m, ro2, cm8) = tq[m] - G[m];  // ((F-F)+G)-G
+            for (int m = 0; m < NV; m++) d[m] = tq[m] - G[m];  // ((F-F)+G)-G
+            store_planes(p.acc, p.plane, ro2, v.cm8, d);
           } else {
+            double a[NV];
+            if constexpr (!ZPRE) load_planes<NV>(p.acc, p.plane, ro2, v.cm8, a);
 #pragma unroll
-            for (int m = 0; m < NV; m++) {
-              double a;
-              if constexpr (ZPRE) a = azp[m];
-              else a = lane_at((const double *)p.acc, plane, m, ro2, cm8);
-              d[m] = a + Gl[m] - G[m];  // (.. + H(k-1)) - H(k)
-            }
+            for (int m = 0; m < NV; m++) d[m] = (ZPRE ? azp[m] : a[m]) + Gl[m] - G[m];  // (.. + H(k-1)) - H(k)
           }
           if constexpr (FINAL) {
             double o9[NV];
             if constexpr (STAGE == 1) {
+              if constexpr (!PREF) {
+                load_planes<4>(p.us, p.plane, ro2, v.cm8, usp);
 #pragma unroll
-              for (int m = 0; m < NV; m++) {
-                double uu;
-                if constexpr (PREF) {
-                  uu = usp[m];  // slot 8 from the ring: glm_f * psi already
-                } else if (m >= 4) {
-                  uu = lds.ring[sa][m][lane + RO];  // as above: slots 4-8 from the ring
-                } else {
-                  uu = lane_at(p.us, plane, m, ro2, cm8);
-                }
-                o9[m] = uu + dtx * d[m];  // rk_tvd21 / rk_std21
+                for (int m = 4; m < NV; m++) usp[m] = lds.ring[sa][m][lane];  // as above
               }
+#pragma unroll
+              for (int m = 0; m < NV; m++) o9[m] = usp[m] + q.dtx * d[m];  // rk_tvd21 / rk_std21
+            } else if constexpr (FOLD) {
+#pragma unroll
+              for (int m = 0; m < NV; m++) o9[m] = 0.5 * (a0p[m] + q.dtx * d[m]);  // rk_tvd22: a0p holds U^n + U*
             } else {
+              if constexpr (!PREF) load_planes<NV>(p.u0, p.plane, ro2, v.cm8, a0p);
+              if constexpr (TT == 0) load_planes<4>(p.us, p.plane, ro2, v.cm8, usp);
 #pragma unroll
               for (int m = 0; m < NV; m++) {
-                if constexpr (FOLD) {
-                  o9[m] = 0.5 * (a0p[m] + dtx * d[m]);  // rk_tvd22: a0p holds U^n + U*
+                double a0 = a0p[m];
+                if (m == 8) a0 = q.glm_f * a0;
+                if constexpr (TT == 0) {  // rk_tvd22; U* slots 4-8 from the ring
+                  const double us = m >= 4 ? lds.ring[sa][m][lane] : usp[m];
+                  o9[m] = 0.5 * (a0 + us + q.dtx * d[m]);
                 } else {
-                  double a0;
-                  if constexpr (PREF) a0 = a0p[m];
-                  else a0 = lane_at(p.u0, plane, m, ro2, cm8);
-                  if (m == 8) a0 = glm_f * a0;
-                  if constexpr (TT == 0) {  // rk_tvd22; U* slots 4-8 from the ring
-                    const double us = m >= 4 ? lds.ring[sa][m][lane + RO] : lane_at(p.us, plane, m, ro2, cm8);
-                    o9[m] = 0.5 * (a0 + us + dtx * d[m]);
-                  } else {
-                    o9[m] = a0 + dtx * d[m];  // rk_std22
-                  }
+                  o9[m] = a0 + q.dtx * d[m];  // rk_std22
                 }
               }
-              o9[8] = glm_f * o9[8];  // glm_ss2 after the step (main.f90:185)
             }
-#pragma unroll
-            for (int m = 0; m < NV; m++) lane_at(p.out, plane, m, ro2, cm8) = o9[m];
-            if constexpr (STAGE == 2) {  // next step's u2v and set_dt on U^{n+1}
-              double w2[NV];
-              cons_to_prim(o9, w2);
-              if (!(w2[3] > 0.0) || !(o9[4] > 0.0))
-                (void)atomicCAS(p.err_next, 0, (w2[3] > 0.0) ? OMHD_ERR_DENSITY : OMHD_ERR_PRESSURE);
-              const double vt = fastest_speed<ND>(o9, w2);
-              vloc = (vt > vloc || !(vt == vt)) ? vt : vloc;
-            }
+            if constexpr (STAGE == 2) o9[8] = q.glm_f * o9[8];  // glm_ss2 after the step (main.f90:185)
+            store_planes(p.out, p.plane, ro2, v.cm8, o9);
+            if constexpr (STAGE == 2) next_speed<ND>(p, o9, vloc);
           }
         }
 #pragma unroll
@@ -568,11 +685,7 @@ __device__ __forceinline__ void march_tile(const Sweep &p, const int t, LdsOf<RE
       }
     }
   }
-  if constexpr (FINAL && STAGE == 2) {
-    if (!(vloc >= 0.0)) (void)atomicCAS(p.err_next + 1, 0, OMHD_ERR_DT);
-    const double vm = wave_max(vloc >= 0.0 ? vloc : 0.0);
-    if (lane == 0) atomic_max_nonneg(p.vmax_bits, vm);
-  }
+  if constexpr (FINAL && STAGE == 2) reduce_speed(p, vloc, lane);
 }
 
 template <int LIM, int STAGE, int TT, int PASS, int RES>
@@ -588,7 +701,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
 // types (p.ftype), same structure
 template <int LIM, int STAGE, int TT, int PASS>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void k_march_gen(const Sweep p) {
-  __shared__ LdsOf<0, PASS_2D> lds;
+  __shared__ SweepLds lds;
   const int t = xcd_remap(blockIdx.x, gridDim.x);
   if (t >= p.ntiles) return;
   if (STAGE == 2 && p.err[0] != 0) return;  // stage 1 failed: leave U^n as it is
@@ -600,7 +713,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
 template <int LIM, int STAGE, int TT>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void k_march_ens(
     const Sweep *__restrict__ members, const int2 *__restrict__ tiles, int ntiles) {
-  __shared__ LdsOf<0, PASS_2D> lds;
+  __shared__ SweepLds lds;
   for (int w = blockIdx.x; w < ntiles; w += gridDim.x) {
     const int2 tl = tiles[w];
     Sweep p = members[tl.x];
@@ -743,11 +856,11 @@ __global__ void k_cfl(const double *__restrict__ s, long long plane, long long z
     double u[NV], w[NV];
 #pragma unroll
     for (int m = 0; m < NV; m++) u[m] = s[m * plane + o];
-    cons_to_prim(u, w);
+    const bool moderate = cons_to_prim(u, w);
     const int kk = ND == 3 ? k + 2 : 0;
     if (!(w[3] > 0.0) || !(u[4] > 0.0))
       record_error(err, (w[3] > 0.0) ? OMHD_ERR_DENSITY : OMHD_ERR_PRESSURE, i + 2, j + 2, kk);
-    const double c = fastest_speed<ND>(u, w);
+    const double c = cell_speed<ND>(u, w, moderate);
     if (!(c >= 0.0)) record_error(err, OMHD_ERR_DT, i + 2, j + 2, kk);
     else vt = dmax(vt, c);
   }
