@@ -34,7 +34,7 @@ struct omhd_handle {
   double vmax = -1.0;  // CFL speed of the current state
   bool have_state = false;
   omhd::Faces faces{};
-  int rows = 24;
+  int rows = 24, rows_z = 24;  // chunk heights of the 2D / XY pass and of the Z pass
   // optional per-stage timing with HIP events on the handle's stream
   bool timing = false;
   hipEvent_t ev[3] = {nullptr, nullptr, nullptr};

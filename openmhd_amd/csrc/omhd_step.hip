@@ -965,28 +965,52 @@ march_fn march_kernel(int pass, int res, int lim, int stage, int tt, bool gen = 
   return res ? pick2<PASS_Z, 1>(lim, stage, tt) : pick2<PASS_Z, 0>(lim, stage, tt);
 }
 
-// Chunk height when the caller leaves it to the library.  Each wavefront
-// marches its chunk row after row, so once a grid has fewer than a few rounds
-// of wavefronts (slots = CUs x 2 per SIMD x 4 SIMDs) the step time follows the
-// chunk height, not the cell count: KH 512^2 ran 2.5x faster with 8-row chunks
-// than with 28.  Such grids take the height that minimises
-// ceil(tiles / slots) * (rows + 3), the 3 being the rows loaded before a chunk's
-// first update (ties to the taller chunk).  Larger grids keep the measured
-// heights: 28 rows in 2D (KH 4096^2), 24 in 3D (Harris 512x256x256).
-int default_rows(int nx, int ny, int nz, int nd, long long slots) {
-  const long long strips = (nx + STRIP - 1) / STRIP, slices = nd == 3 ? nz : 1;
-  auto tiles = [&](int r) { return strips * slices * ((ny + r - 1) / r); };
+// Time of one pass over `tiles` chunks of r rows, in microseconds, as measured
+// for the 2D pass (both stages' mean, KH and Orszag-Tang grids of 64^2 to
+// 4096^2, heights 1 to 56: within 10% but for grids of many rounds, where the
+// rounds blur).  Two wavefronts share a SIMD (`slots` of them in all): a chunk
+// then takes 8.5 + 7 r, against 6 + 4.8 r for one that has the SIMD to itself,
+// and full rounds of `slots` chunks follow each other.  The 8.5 is what a
+// chunk pays before its first updated row (one load latency and two flux
+// evaluations).  3D passes scale alike, so the same line serves.
+double march_cost(long long tiles, int r, long long slots) {
+  const long long full = tiles / slots, rest = tiles % slots;
+  const double shared = 8.5 + 7.0 * r, alone = 6.0 + 4.8 * r;
+  return (double)full * shared + (rest == 0 ? 0.0 : (2 * rest <= slots ? alone : shared));
+}
+
+// Chunk height when the caller leaves it to the library: the one of least
+// march_cost, from 1 row up (a lone wavefront marches its rows one after the
+// other at 4.8 us each, so a small grid wants as many chunks as the chip has
+// room for: KH 64^2 runs a stage in 15 us with 1-row chunks and 49 with 8;
+// 512^2 in 39 us with 5 rows, 51 with 8; 1448^2 in 152 us with 18, 208 with
+// 28).  Grids of four rounds and more keep the heights measured best for them
+// (KH 4096^2: 28 rows; Harris 512x256x256: 24, where 10 to 28 are within 2%).
+// `tiles(r)`: the pass's number of chunks of r rows; nm: its rows.
+template <class Tiles>
+int default_rows(const Tiles &tiles, int nm, int nd, long long slots) {
   if (tiles(24) >= 4 * slots) return nd == 2 ? 28 : 24;
-  int best = 28;
-  long long best_cost = -1;
-  for (int r : {28, 24, 20, 16, 12, 8}) {
-    const long long cost = (tiles(r) + slots - 1) / slots * (r + 3);
-    if (best_cost < 0 || cost < best_cost) {
+  int best = 1;
+  double best_cost = 0.0;
+  for (int r = 1; r <= 28 && r <= nm; r++) {
+    const double cost = march_cost(tiles(r), r, slots);
+    if (r == 1 || cost <= best_cost) {
       best_cost = cost;
       best = r;
     }
   }
   return best;
+}
+
+// wavefront slots of the current device: CUs x 4 SIMDs x 2
+long long march_slots() {
+  int dev = 0, cus = 256;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1) {
+    (void)hipGetLastError();
+    cus = 256;
+  }
+  return 8LL * cus;
 }
 
 unsigned sign_mask(const double *s9) {
@@ -1063,18 +1087,15 @@ extern "C" int omhd_create(const omhd_config *cfg, omhd_handle **out) {
   h->pitch = (cfg->nx + 7) & ~7;  // 64-byte aligned rows
   h->zstride = (long long)h->pitch * cfg->ny;
   h->plane = ((h->zstride * nz) + 63) & ~63LL;
-  // default chunk heights (default_rows), measured: on KH 4096^2, chunks of 16,
-  // 24 or 32 rows ran about 2% slower than 20 or 28 (28 best); on the
-  // 512x256x256 Harris sheet 24 was best, with 20 and 28 within 0.5%
   if (cfg->rows_per_wave > 0) {
-    h->rows = cfg->rows_per_wave;
+    h->rows = h->rows_z = cfg->rows_per_wave;
   } else {
-    int dev = 0, cus = 256;
-    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1) {
-      (void)hipGetLastError();
-      cus = 256;
-    }
-    h->rows = default_rows(cfg->nx, cfg->ny, nz, cfg->ndim, 8LL * cus);
+    const long long slots = march_slots(), strips = (cfg->nx + STRIP - 1) / STRIP;
+    const long long slices = cfg->ndim == 3 ? nz : 1;
+    // the resistive XY pass's LDS leaves room for 7 wavefronts per CU, not 8
+    h->rows = default_rows([&](int r) { return strips * slices * ((cfg->ny + r - 1) / r); }, cfg->ny, cfg->ndim,
+                           cfg->resistive ? slots / 8 * 7 : slots);
+    h->rows_z = default_rows([&](int r) { return strips * cfg->ny * (long long)((nz + r - 1) / r); }, nz, 3, slots);
   }
   for (int a = 0; a < 3; a++) {
     h->faces.bc[a] = cfg->bc_type[2 * a];
@@ -1322,7 +1343,7 @@ static Sweep base_sweep(omhd_handle *h, int pass) {
   p.ny = c.ny;
   p.nz = c.nz;
   p.nstrip = (c.nx + STRIP - 1) / STRIP;
-  p.rows = h->rows;
+  p.rows = pass == PASS_Z ? h->rows_z : h->rows;
   const int nm = pass == PASS_Z ? c.nz : c.ny;
   const int nslice = pass == PASS_2D ? 1 : pass == PASS_XY ? c.nz : c.ny;
   p.nchunk = (nm + p.rows - 1) / p.rows;
@@ -1849,10 +1870,16 @@ extern "C" int omhd_batch_create(const omhd_config *cfgs, int32_t n, omhd_batch 
   }
   OMHD_HIP(hipMemset(b->err_d, 0, 8 * sizeof(int)));
   OMHD_HIP(hipMemset(b->tsum_d, 0, n * sizeof(double)));
+  int ny_max = 0;
+  for (const Sweep &p : b->mem) ny_max = std::max(ny_max, p.ny);
+  b->rows = default_rows(
+      [&](int r) {
+        long long t = 0;
+        for (const Sweep &p : b->mem) t += (long long)p.nstrip * ((p.ny + r - 1) / r);
+        return t;
+      },
+      ny_max, 2, march_slots());
   if (int rc = batch_tiles(b)) return rc;
-  int dev = 0, cus = 256;
-  (void)hipGetDevice(&dev);
-  (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
   b->grid = 0;  // 0: one workgroup per tile; >0: persistent grid of that many workgroups
   *out = b;
   return ok();
