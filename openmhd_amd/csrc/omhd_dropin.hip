@@ -154,34 +154,67 @@ __global__ __launch_bounds__(256) void k_u2v(const double *__restrict__ U, doubl
 }
 
 // ---------------------------------------------------------------------------
-// limiter along one direction (limiter.f90).  Lines run along `dir` with
-// stride s and length nl; (a, b) enumerate the transverse ranges.
+// The cells (or faces) of a kernel: (ni, nj, nk) of them from (i0, j0, k0) of
+// an array, x fastest, so that a wavefront's accesses are contiguous whatever
+// the kernel's direction.
+// ---------------------------------------------------------------------------
+struct Box {
+  int i0, ni, j0, nj, k0, nk;
+  __host__ __device__ size_t count() const { return (size_t)(ni > 0 ? ni : 0) * (nj > 0 ? nj : 0) * (nk > 0 ? nk : 0); }
+};
+// cell number gid, false past the last.  Indices are split with 32-bit
+// divisions where the count allows (a 64-bit division is some hundred
+// instructions, more than most of these kernels have).
+__device__ __forceinline__ bool cell_of(const Box &b, size_t gid, int &i, int &j, int &k) {
+  const size_t n = b.count();
+  if (gid >= n) return false;
+  if (n <= 0xffffffffull) {
+    const unsigned g = (unsigned)gid, r = g / (unsigned)b.ni;
+    i = b.i0 + (int)(g - r * (unsigned)b.ni);
+    const unsigned q = r / (unsigned)b.nj;
+    j = b.j0 + (int)(r - q * (unsigned)b.nj);
+    k = b.k0 + (int)q;
+  } else {
+    const size_t r = gid / b.ni, q = r / b.nj;
+    i = b.i0 + (int)(gid - r * b.ni);
+    j = b.j0 + (int)(r - q * b.nj);
+    k = b.k0 + (int)q;
+  }
+  return true;
+}
+__device__ __forceinline__ size_t thread_number() { return (size_t)blockIdx.x * blockDim.x + threadIdx.x; }
+
+// ---------------------------------------------------------------------------
+// limiter along one direction (limiter.f90): one lane per cell of the box,
+// whose extent along `dir` is the whole line of nl cells, stride s.  Bound by
+// memory (24 B per cell).  With lanes along the line, as the loop reads, the
+// lanes of a y or z line were ix apart: 52 us a call on 160x128x120 cells over
+// the three directions; 16.5 us in this
+// order (59 MB, 3.6 TB/s).
 // ---------------------------------------------------------------------------
 template <int T>
-__global__ __launch_bounds__(256) void k_limiter(const double *__restrict__ wk, double *__restrict__ wL, double *__restrict__ wR, int nl,
-                          size_t s, int na, int nb, size_t sa, size_t sb, size_t base) {
-  size_t gid = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  size_t total = (size_t)nl * na * nb;
-  if (gid >= total) return;
-  const int l = (int)(gid % nl);  // 0-based position on the line
-  const size_t r = gid / nl;
-  const int a = (int)(r % na), b = (int)(r / na);
-  const size_t o = base + (size_t)a * sa + (size_t)b * sb;
+__global__ __launch_bounds__(256) void k_limiter(const double *__restrict__ wk, double *__restrict__ wL,
+                                                 double *__restrict__ wR, const Box b, int ix, int jx, int dir, int nl,
+                                                 size_t s) {
+  int i, j, k;
+  if (!cell_of(b, thread_number(), i, j, k)) return;
+  const size_t c = (size_t)i + (size_t)ix * ((size_t)j + (size_t)jx * k);
+  const int l = dir == 1 ? i : dir == 2 ? j : k;  // 0-based position on the line
   if constexpr (T == 0) {  // limiter.f90:56-70
     if (l < nl - 1) {
-      wL[o + l * s] = wk[o + l * s];
-      wR[o + l * s] = wk[o + (l + 1) * s];
+      wL[c] = wk[c];
+      wR[c] = wk[c + s];
     }
   } else {
     if (l == 0) {
-      wL[o] = wk[o];
+      wL[c] = wk[c];
     } else if (l == nl - 1) {
-      wR[o + (size_t)(nl - 2) * s] = wk[o + (size_t)(nl - 1) * s];
+      wR[c - s] = wk[c];
     } else {
       double gR, gL;
-      limit<T>(wk[o + (l - 1) * s], wk[o + l * s], wk[o + (l + 1) * s], gR, gL);
-      wR[o + (l - 1) * s] = gR;
-      wL[o + l * s] = gL;
+      limit<T>(wk[c - s], wk[c], wk[c + s], gR, gL);
+      wR[c - s] = gR;
+      wL[c] = gL;
     }
   }
 }
@@ -189,24 +222,31 @@ __global__ __launch_bounds__(256) void k_limiter(const double *__restrict__ wk, 
 // ---------------------------------------------------------------------------
 // HLLD flux at every interface of the reference's loop range
 // ---------------------------------------------------------------------------
+// One lane per cell of F: the faces of the loop range get the flux, the rest
+// of F is zero (flux_solver.f90:57 zeroes F first; writing the zeros here
+// saves a pass over F).  Bound by memory, 216 B per cell: 160x128x120 cells
+// 113 to 124 us (4.3 to 4.7 TB/s), 125 us and a fill of 38 us before.
 template <int D>
-__global__ __launch_bounds__(256) void k_flux(double *__restrict__ F, const double *__restrict__ VL, const double *__restrict__ VR, double ch,
-                       int ix, int jx, int kx, int i0, int ni, int j0, int nj, int k0, int nk, int type) {
-  size_t gid = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (gid >= (size_t)ni * nj * nk) return;
-  const int i = i0 + (int)(gid % ni);
-  const size_t r = gid / ni;
-  const int j = j0 + (int)(r % nj), k = k0 + (int)(r / nj);
-  const size_t n = (size_t)ix * jx * kx;
-  const size_t c = (size_t)i + (size_t)ix * ((size_t)j + (size_t)jx * k);
-  double L[NV], R[NV], f[NV];
+__global__ __launch_bounds__(256) void k_flux(double *__restrict__ F, const double *__restrict__ VL,
+                                              const double *__restrict__ VR, double ch, const Box all, const Box b,
+                                              int type) {
+  int i, j, k;
+  if (!cell_of(all, thread_number(), i, j, k)) return;
+  const size_t n = all.count();
+  const size_t c = (size_t)i + (size_t)all.ni * ((size_t)j + (size_t)all.nj * k);
+  double f[NV];
 #pragma unroll
-  for (int m = 0; m < NV; m++) {
-    L[m] = VL[m * n + c];
-    R[m] = VR[m * n + c];
+  for (int m = 0; m < NV; m++) f[m] = 0.0;
+  if (i >= b.i0 && i < b.i0 + b.ni && j >= b.j0 && j < b.j0 + b.nj && k >= b.k0 && k < b.k0 + b.nk) {
+    double L[NV], R[NV];
+#pragma unroll
+    for (int m = 0; m < NV; m++) {
+      L[m] = VL[m * n + c];
+      R[m] = VR[m * n + c];
+    }
+    if (type == 3) hlld<D>(L, R, ch, ch * ch, f, moderate_pair(L, R));
+    else riemann_other<D>(type, L, R, ch, ch * ch, f);
   }
-  if (type == 3) hlld<D>(L, R, ch, ch * ch, f, moderate_pair(L, R));
-  else riemann_other<D>(type, L, R, ch, ch * ch, f);
 #pragma unroll
   for (int m = 0; m < NV; m++) F[m * n + c] = f[m];
 }
@@ -221,12 +261,8 @@ __global__ void k_scale(double *__restrict__ a, double f, size_t n) {
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void k_rk(int mode, double *__restrict__ wk, double *__restrict__ wk1, const double *__restrict__ wF,
                      const double *__restrict__ wG, const double *__restrict__ wH, double dtx, int ix, int jx, int kx) {
-  const int ni = ix - 2, nj = jx - 2, nk = wH ? kx - 2 : 1;
-  size_t gid = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (gid >= (size_t)ni * nj * nk) return;
-  const int i = 1 + (int)(gid % ni);
-  const size_t r = gid / ni;
-  const int j = 1 + (int)(r % nj), k = (wH ? 1 : 0) + (int)(r / nj);
+  int i, j, k;
+  if (!cell_of(Box{1, ix - 2, 1, jx - 2, wH ? 1 : 0, wH ? kx - 2 : 1}, thread_number(), i, j, k)) return;
   const size_t n = (size_t)ix * jx * kx;
   const size_t c = (size_t)i + (size_t)ix * ((size_t)j + (size_t)jx * k);
   const size_t sj = ix, sk = (size_t)ix * jx;
@@ -240,49 +276,26 @@ __global__ __launch_bounds__(256) void k_rk(int mode, double *__restrict__ wk, d
   }
 }
 
-// ---------------------------------------------------------------------------
-// set_dt: per-cell fastest speed, wave max, one atomic per wave
-// ---------------------------------------------------------------------------
-template <int ND>
-__global__ __launch_bounds__(256) void k_speed(const double *__restrict__ U, const double *__restrict__ V, int ix, int jx, int kx,
-                        unsigned long long *vmax_bits, int *flags) {
-  const int is = ix > 1 ? 1 : 0, js = jx > 1 ? 1 : 0, ks = kx > 1 ? 1 : 0;
-  const int ni = ix > 2 ? ix - 2 : 1, nj = jx > 2 ? jx - 2 : 1, nk = kx > 2 ? kx - 2 : 1;
-  size_t gid = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  double vt = 0.0;
-  if (gid < (size_t)ni * nj * nk) {
-    const int i = is + (int)(gid % ni);
-    const size_t r = gid / ni;
-    const int j = js + (int)(r % nj), k = ks + (int)(r / nj);
-    const size_t n = (size_t)ix * jx * kx;
-    const size_t c = (size_t)i + (size_t)ix * ((size_t)j + (size_t)jx * k);
-    double u[NV], w[NV];
-#pragma unroll
-    for (int m = 0; m < NV; m++) u[m] = U[m * n + c];
-#pragma unroll
-    for (int m = 0; m < 4; m++) w[m] = V[m * n + c];
-    vt = fastest_speed<ND>(u, w);
-    if (!(vt >= 0.0)) atomicOr(flags, 4);  // NaN
-  }
-  vt = wave_max(vt);
-  if ((threadIdx.x & 63) == 0) atomic_max_nonneg(vmax_bits, vt);
+// interior cells as set_dt counts them (an extent of 1 or 2 counts one)
+__host__ __device__ __forceinline__ Box speed_box(int ix, int jx, int kx) {
+  auto lo = [](int e) { return e > 1 ? 1 : 0; };
+  auto num = [](int e) { return e > 2 ? e - 2 : 1; };
+  return Box{lo(ix), num(ix), lo(jx), num(jx), lo(kx), num(kx)};
 }
-
-// ---------------------------------------------------------------------------
-// set_dt without allocation (omhd_set_dt_noalloc).  The scratch array holds
-// one partial per workgroup: pass 1 has each workgroup take
-// NOALLOC_CELLS_PER_GROUP interior cells and store its maximum speed and its
-// flags in its own slots; pass 2, one workgroup, reduces the slots of the
-// workgroups pass 1 ran.  Every slot a call reads is written earlier in the
-// same call, so nothing needs clearing, and no atomics are used.
-// ---------------------------------------------------------------------------
-constexpr int NOALLOC_GROUPS = 32768;
-constexpr int NOALLOC_CELLS_PER_THREAD = 8;
-constexpr size_t NOALLOC_CELLS_PER_GROUP = (size_t)TPB * NOALLOC_CELLS_PER_THREAD;
-constexpr size_t NOALLOC_MAX_CELLS = (size_t)NOALLOC_GROUPS * NOALLOC_CELLS_PER_GROUP;  // 67,108,864
-// [0, G): max-speed bits per workgroup; [G, 2G): flags per workgroup;
-// [2G], [2G+1]: the reduced max-speed bits and flags.  512 KiB + 16 B per GPU.
-__device__ __align__(256) unsigned long long scratch[2 * NOALLOC_GROUPS + 2];
+// fastest speed of cell number gid of the box
+template <int ND>
+__device__ __forceinline__ double speed_at(const double *__restrict__ U, const double *__restrict__ V, const Box &b,
+                                           size_t gid, int ix, int jx, size_t n) {
+  int i, j, k;
+  (void)cell_of(b, gid, i, j, k);
+  const size_t c = (size_t)i + (size_t)ix * ((size_t)j + (size_t)jx * k);
+  double u[NV], w[NV];
+#pragma unroll
+  for (int m = 0; m < NV; m++) u[m] = U[m * n + c];
+#pragma unroll
+  for (int m = 0; m < 4; m++) w[m] = V[m * n + c];
+  return fastest_speed<ND>(u, w);
+}
 
 // workgroup-wide max of non-negative doubles and OR of flags (TPB threads)
 __device__ __forceinline__ void group_reduce(double &v, int &f) {
@@ -303,27 +316,63 @@ __device__ __forceinline__ void group_reduce(double &v, int &f) {
     }
 }
 
+// ---------------------------------------------------------------------------
+// set_dt: per-cell fastest speed, one atomic per workgroup.  SPEED_GROUPS
+// workgroups at most, each over many cells: the atomics and the reads before
+// them all go to one address, so their number is bounded, and 2048 workgroups
+// fill the chip.  Bound by memory (64 B per cell).  160x128x120 cells: 40 us,
+// 105 us with a workgroup per 256 cells and an atomic per wavefront.
+// ---------------------------------------------------------------------------
+constexpr unsigned SPEED_GROUPS = 2048;
+template <int ND>
+__global__ __launch_bounds__(256) void k_speed(const double *__restrict__ U, const double *__restrict__ V, int ix, int jx, int kx,
+                        unsigned long long *vmax_bits, int *flags) {
+  const Box b = speed_box(ix, jx, kx);
+  const size_t total = b.count(), n = (size_t)ix * jx * kx, step = (size_t)gridDim.x * blockDim.x;
+  double vt = 0.0;
+  int f = 0;
+  for (size_t gid = thread_number(); gid < total; gid += step) {
+    const double v = speed_at<ND>(U, V, b, gid, ix, jx, n);
+    const bool bad = !(v >= 0.0);  // NaN: flagged; vmax is NaN if it fills a wavefront's 64 cells
+    if (bad) f |= 4;
+    if (__builtin_amdgcn_ballot_w64(bad) == ~0ull) f |= 8;
+    vt = dmax(vt, v);
+  }
+  group_reduce(vt, f);
+  if (threadIdx.x == 0) {
+    if (f & 8) vt = __builtin_nan("");
+    if (f) atomicOr(flags, 4);
+    atomic_max_nonneg(vmax_bits, vt);
+  }
+}
+
+// ---------------------------------------------------------------------------
+// set_dt without allocation (omhd_set_dt_noalloc).  The scratch array holds
+// one partial per workgroup: pass 1 has each workgroup take
+// NOALLOC_CELLS_PER_GROUP interior cells and store its maximum speed and its
+// flags in its own slots; pass 2, one workgroup, reduces the slots of the
+// workgroups pass 1 ran.  Every slot a call reads is written earlier in the
+// same call, so nothing needs clearing, and no atomics are used.
+// ---------------------------------------------------------------------------
+constexpr int NOALLOC_GROUPS = 32768;
+constexpr int NOALLOC_CELLS_PER_THREAD = 8;
+constexpr size_t NOALLOC_CELLS_PER_GROUP = (size_t)TPB * NOALLOC_CELLS_PER_THREAD;
+constexpr size_t NOALLOC_MAX_CELLS = (size_t)NOALLOC_GROUPS * NOALLOC_CELLS_PER_GROUP;  // 67,108,864
+// [0, G): max-speed bits per workgroup; [G, 2G): flags per workgroup;
+// [2G], [2G+1]: the reduced max-speed bits and flags.  512 KiB + 16 B per GPU.
+__device__ __align__(256) unsigned long long scratch[2 * NOALLOC_GROUPS + 2];
+
 template <int ND>
 __global__ __launch_bounds__(256) void k_speed_part(const double *__restrict__ U, const double *__restrict__ V, int ix,
                                                     int jx, int kx, unsigned long long *part) {
-  const int is = ix > 1 ? 1 : 0, js = jx > 1 ? 1 : 0, ks = kx > 1 ? 1 : 0;
-  const int ni = ix > 2 ? ix - 2 : 1, nj = jx > 2 ? jx - 2 : 1, nk = kx > 2 ? kx - 2 : 1;
-  const size_t total = (size_t)ni * nj * nk, n = (size_t)ix * jx * kx;
+  const Box b = speed_box(ix, jx, kx);
+  const size_t total = b.count(), n = (size_t)ix * jx * kx;
   double vt = 0.0;
   int f = 0;
   for (int q = 0; q < NOALLOC_CELLS_PER_THREAD; q++) {
     const size_t gid = (size_t)blockIdx.x * NOALLOC_CELLS_PER_GROUP + (size_t)q * TPB + threadIdx.x;
     if (gid >= total) break;
-    const int i = is + (int)(gid % ni);
-    const size_t r = gid / ni;
-    const int j = js + (int)(r % nj), k = ks + (int)(r / nj);
-    const size_t c = (size_t)i + (size_t)ix * ((size_t)j + (size_t)jx * k);
-    double u[NV], w[NV];
-#pragma unroll
-    for (int m = 0; m < NV; m++) u[m] = U[m * n + c];
-#pragma unroll
-    for (int m = 0; m < 4; m++) w[m] = V[m * n + c];
-    const double c1 = fastest_speed<ND>(u, w);
+    const double c1 = speed_at<ND>(U, V, b, gid, ix, jx, n);
     if (!(c1 >= 0.0)) f |= 4;  // NaN
     else vt = dmax(vt, c1);
   }
@@ -350,67 +399,67 @@ __global__ __launch_bounds__(256) void k_speed_final(const unsigned long long *_
 }
 
 // ---------------------------------------------------------------------------
-// ghost fill, one face pair per launch (x, then y, then z: bc.f90 order)
+// ghost fill, one face pair per launch (x, then y, then z: bc.f90 order), and
+// the periodic or wall states of a face pair.  One lane per line along `dir`
+// and component (blockIdx.y): nothing but the latency of a load and a store,
+// which one lane for all nine components paid nine times (15 us a face pair on
+// 160x128x120 cells; 8 us in this form).
 // ---------------------------------------------------------------------------
-__global__ void k_bc_face_pair(double *__restrict__ U, int ix, int jx, int kx, int dir, int type_lo, int type_hi,
-                               const double sl0, const double sl1, const double sl2, const double sl3, const double sl4,
-                               const double sl5, const double sl6, const double sl7, const double sl8, const double sh0,
-                               const double sh1, const double sh2, const double sh3, const double sh4, const double sh5,
-                               const double sh6, const double sh7, const double sh8) {
-  // transverse plane enumeration
-  const int na = (dir == 1) ? jx : ix, nb = (dir == 3) ? jx : kx;
-  size_t gid = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (gid >= (size_t)na * nb) return;
-  const int a = (int)(gid % na), b = (int)(gid / na);
-  const size_t n = (size_t)ix * jx * kx;
-  size_t base, s;
-  int nl;
-  if (dir == 1) { base = (size_t)ix * ((size_t)a + (size_t)jx * b); s = 1; nl = ix; }
-  else if (dir == 2) { base = (size_t)a + (size_t)ix * (size_t)jx * b; s = ix; nl = jx; }
-  else { base = (size_t)a + (size_t)ix * b; s = (size_t)ix * jx; nl = kx; }
-  const double sl[NV] = {sl0, sl1, sl2, sl3, sl4, sl5, sl6, sl7, sl8};
-  const double sh[NV] = {sh0, sh1, sh2, sh3, sh4, sh5, sh6, sh7, sh8};
-  for (int m = 0; m < NV; m++) {
-    double *A = U + m * n + base;
-    if (type_lo == OMHD_BC_PERIODIC) {  // bc.f90:9-14 (high side first)
-      A[(size_t)(nl - 1) * s] = A[s];
-      A[0] = A[(size_t)(nl - 2) * s];
-    } else {
-      A[0] = sl[m] * A[s];
-      A[(size_t)(nl - 1) * s] = sh[m] * A[(size_t)(nl - 2) * s];
-    }
-  }
-  (void)type_hi;
+struct Signs {
+  double lo[NV], hi[NV];
+};
+// element number of line gid's first cell along dir, its stride and length
+__device__ __forceinline__ bool line_of(size_t gid, int ix, int jx, int kx, int dir, size_t &base, size_t &s, int &nl) {
+  int i, j, k;
+  if (!cell_of(Box{0, dir == 1 ? 1 : ix, 0, dir == 2 ? 1 : jx, 0, dir == 3 ? 1 : kx}, gid, i, j, k)) return false;
+  base = (size_t)i + (size_t)ix * ((size_t)j + (size_t)jx * k);
+  s = dir == 1 ? 1 : dir == 2 ? (size_t)ix : (size_t)ix * jx;
+  nl = dir == 1 ? ix : dir == 2 ? jx : kx;
+  return true;
 }
 
-__global__ void k_face_patch(double *__restrict__ VL, double *__restrict__ VR, int ix, int jx, int kx, int dir,
-                             int type, const double sl0, const double sl1, const double sl2, const double sl3,
-                             const double sl4, const double sl5, const double sl6, const double sl7, const double sl8,
-                             const double sh0, const double sh1, const double sh2, const double sh3, const double sh4,
-                             const double sh5, const double sh6, const double sh7, const double sh8) {
-  const int na = (dir == 1) ? jx : ix, nb = (dir == 3) ? jx : kx;
-  size_t gid = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (gid >= (size_t)na * nb) return;
-  const int a = (int)(gid % na), b = (int)(gid / na);
-  const size_t n = (size_t)ix * jx * kx;
+__global__ __launch_bounds__(256) void k_bc_face_pair(double *__restrict__ U, int ix, int jx, int kx, int dir, int type_lo,
+                                                      const Signs sg) {
   size_t base, s;
   int nl;
-  if (dir == 1) { base = (size_t)ix * ((size_t)a + (size_t)jx * b); s = 1; nl = ix; }
-  else if (dir == 2) { base = (size_t)a + (size_t)ix * (size_t)jx * b; s = ix; nl = jx; }
-  else { base = (size_t)a + (size_t)ix * b; s = (size_t)ix * jx; nl = kx; }
-  const double sl[NV] = {sl0, sl1, sl2, sl3, sl4, sl5, sl6, sl7, sl8};
-  const double sh[NV] = {sh0, sh1, sh2, sh3, sh4, sh5, sh6, sh7, sh8};
-  const size_t lo = base, hi = base + (size_t)(nl - 2) * s;
-  for (int m = 0; m < NV; m++) {
-    double *L = VL + m * n, *R = VR + m * n;
-    if (type == OMHD_BC_PERIODIC) {  // main.f90:101-102
-      R[hi] = R[lo];
-      L[lo] = L[hi];
-    } else {  // 2D_KH/bc.f90:61-81
-      L[lo] = sl[m] * R[lo];
-      R[hi] = sh[m] * L[hi];
-    }
+  if (!line_of(thread_number(), ix, jx, kx, dir, base, s, nl)) return;
+  const int m = blockIdx.y;
+  double *A = U + (size_t)m * ix * jx * kx + base;
+  if (type_lo == OMHD_BC_PERIODIC) {  // bc.f90:9-14 (high side first)
+    A[(size_t)(nl - 1) * s] = A[s];
+    A[0] = A[(size_t)(nl - 2) * s];
+  } else {
+    A[0] = sg.lo[m] * A[s];
+    A[(size_t)(nl - 1) * s] = sg.hi[m] * A[(size_t)(nl - 2) * s];
   }
+}
+
+__global__ __launch_bounds__(256) void k_face_patch(double *__restrict__ VL, double *__restrict__ VR, int ix, int jx,
+                                                    int kx, int dir, int type, const Signs sg) {
+  size_t base, s;
+  int nl;
+  if (!line_of(thread_number(), ix, jx, kx, dir, base, s, nl)) return;
+  const int m = blockIdx.y;
+  const size_t o = (size_t)m * ix * jx * kx + base, last = (size_t)(nl - 2) * s;
+  double *L = VL + o, *R = VR + o;
+  if (type == OMHD_BC_PERIODIC) {  // main.f90:101-102
+    R[last] = R[0];
+    L[0] = L[last];
+  } else {  // 2D_KH/bc.f90:61-81
+    L[0] = sg.lo[m] * R[0];
+    R[last] = sg.hi[m] * L[last];
+  }
+}
+
+static Signs signs(const double *lo, const double *hi) {
+  Signs g;
+  memcpy(g.lo, lo, sizeof g.lo);
+  memcpy(g.hi, hi, sizeof g.hi);
+  return g;
+}
+// a face pair's launch: (lines, components)
+static dim3 face_grid(int ix, int jx, int kx, int dir) {
+  return dim3(nblocks((size_t)(dir == 1 ? jx : ix) * (dir == 3 ? jx : kx)), NV);
 }
 
 // 2D_reconnection/flux_resistive.f90:66-111, the 2D CPU form of the resistive
@@ -623,33 +672,21 @@ extern "C" int omhd_limiter(const double *wk, double *wL, double *wR, int32_t ix
   if (int rc = br.init(wR, n, true, true, s)) return rc;
   auto lo = [](int e) { return e < 2 ? e : 2; };
   auto hi = [](int e) { return e - 1 > 1 ? e - 1 : 1; };
-  int nl, na, nb;
-  size_t st, sa, sb, base;
   const size_t sj = ix, sk = (size_t)ix * jx;
-  if (dir == 1) {
-    nl = ix; st = 1;
-    na = hi(jx) - lo(jx) + 1; sa = sj;
-    nb = hi(kx) - lo(kx) + 1; sb = sk;
-    base = (size_t)(lo(jx) - 1) * sj + (size_t)(lo(kx) - 1) * sk;
-  } else if (dir == 2) {
-    nl = jx; st = sj;
-    na = hi(ix) - lo(ix) + 1; sa = 1;
-    nb = hi(kx) - lo(kx) + 1; sb = sk;
-    base = (size_t)(lo(ix) - 1) + (size_t)(lo(kx) - 1) * sk;
-  } else {
-    nl = kx; st = sk;
-    na = hi(ix) - lo(ix) + 1; sa = 1;
-    nb = hi(jx) - lo(jx) + 1; sb = sj;
-    base = (size_t)(lo(ix) - 1) + (size_t)(lo(jx) - 1) * sj;
-  }
-  const size_t total = (size_t)nl * na * nb;
+  Box b{lo(ix) - 1, hi(ix) - lo(ix) + 1, lo(jx) - 1, hi(jx) - lo(jx) + 1, lo(kx) - 1, hi(kx) - lo(kx) + 1};
+  int nl;
+  size_t st;
+  if (dir == 1) { b.i0 = 0; b.ni = nl = ix; st = 1; }
+  else if (dir == 2) { b.j0 = 0; b.nj = nl = jx; st = sj; }
+  else { b.k0 = 0; b.nk = nl = kx; st = sk; }
+  const size_t total = b.count();
   if (nl >= 2 && total > 0) {
     switch (type) {
-      case 0: k_limiter<0><<<nblocks(total), TPB, 0, s>>>(a.dev, bl.dev, br.dev, nl, st, na, nb, sa, sb, base); break;
-      case 1: k_limiter<1><<<nblocks(total), TPB, 0, s>>>(a.dev, bl.dev, br.dev, nl, st, na, nb, sa, sb, base); break;
-      case 2: k_limiter<2><<<nblocks(total), TPB, 0, s>>>(a.dev, bl.dev, br.dev, nl, st, na, nb, sa, sb, base); break;
-      case 3: k_limiter<3><<<nblocks(total), TPB, 0, s>>>(a.dev, bl.dev, br.dev, nl, st, na, nb, sa, sb, base); break;
-      default: k_limiter<4><<<nblocks(total), TPB, 0, s>>>(a.dev, bl.dev, br.dev, nl, st, na, nb, sa, sb, base); break;
+      case 0: k_limiter<0><<<nblocks(total), TPB, 0, s>>>(a.dev, bl.dev, br.dev, b, ix, jx, dir, nl, st); break;
+      case 1: k_limiter<1><<<nblocks(total), TPB, 0, s>>>(a.dev, bl.dev, br.dev, b, ix, jx, dir, nl, st); break;
+      case 2: k_limiter<2><<<nblocks(total), TPB, 0, s>>>(a.dev, bl.dev, br.dev, b, ix, jx, dir, nl, st); break;
+      case 3: k_limiter<3><<<nblocks(total), TPB, 0, s>>>(a.dev, bl.dev, br.dev, b, ix, jx, dir, nl, st); break;
+      default: k_limiter<4><<<nblocks(total), TPB, 0, s>>>(a.dev, bl.dev, br.dev, b, ix, jx, dir, nl, st); break;
     }
     OMHD_HIP(hipGetLastError());
   }
@@ -674,21 +711,17 @@ extern "C" int omhd_flux_solver(double *F, const double *VL, const double *VR, d
   if (int rc = f.init(F, 9 * n, false, true, s)) return rc;
   if (int rc = l.init(VL, 9 * n, true, false, s)) return rc;
   if (int rc = r.init(VR, 9 * n, true, false, s)) return rc;
-  OMHD_HIP(hipMemsetAsync(f.dev, 0, 9 * n * sizeof(double), s));  // flux_solver.f90:57
   auto lo = [](int e) { return e < 2 ? e : 2; };
   auto hi = [](int e) { return e - 1 > 1 ? e - 1 : 1; };
-  int i0 = lo(ix) - 1, ni = hi(ix) - lo(ix) + 1, j0 = lo(jx) - 1, nj = hi(jx) - lo(jx) + 1, k0 = lo(kx) - 1,
-      nk = hi(kx) - lo(kx) + 1;
-  if (dir == 1) { i0 = 0; ni = ix - 1; }
-  if (dir == 2) { j0 = 0; nj = jx - 1; }
-  if (dir == 3) { k0 = 0; nk = kx - 1; }
-  const size_t total = (size_t)(ni > 0 ? ni : 0) * nj * nk;
-  if (total > 0) {
-    if (dir == 1) k_flux<0><<<nblocks(total), TPB, 0, s>>>(f.dev, l.dev, r.dev, ch, ix, jx, kx, i0, ni, j0, nj, k0, nk, type);
-    if (dir == 2) k_flux<1><<<nblocks(total), TPB, 0, s>>>(f.dev, l.dev, r.dev, ch, ix, jx, kx, i0, ni, j0, nj, k0, nk, type);
-    if (dir == 3) k_flux<2><<<nblocks(total), TPB, 0, s>>>(f.dev, l.dev, r.dev, ch, ix, jx, kx, i0, ni, j0, nj, k0, nk, type);
-    OMHD_HIP(hipGetLastError());
-  }
+  const Box all{0, ix, 0, jx, 0, kx};
+  Box b{lo(ix) - 1, hi(ix) - lo(ix) + 1, lo(jx) - 1, hi(jx) - lo(jx) + 1, lo(kx) - 1, hi(kx) - lo(kx) + 1};
+  if (dir == 1) { b.i0 = 0; b.ni = ix - 1; }
+  if (dir == 2) { b.j0 = 0; b.nj = jx - 1; }
+  if (dir == 3) { b.k0 = 0; b.nk = kx - 1; }
+  if (dir == 1) k_flux<0><<<nblocks(n), TPB, 0, s>>>(f.dev, l.dev, r.dev, ch, all, b, type);
+  if (dir == 2) k_flux<1><<<nblocks(n), TPB, 0, s>>>(f.dev, l.dev, r.dev, ch, all, b, type);
+  if (dir == 3) k_flux<2><<<nblocks(n), TPB, 0, s>>>(f.dev, l.dev, r.dev, ch, all, b, type);
+  OMHD_HIP(hipGetLastError());
   if (int rc = f.finish(s)) return rc;
   f.release(s);
   l.release(s);
@@ -757,12 +790,11 @@ extern "C" int omhd_set_dt(const double *U, const double *V, double *vmax, doubl
   unsigned long long *red;
   OMHD_HIP(hipMallocAsync((void **)&red, 2 * sizeof(unsigned long long), s));
   OMHD_HIP(hipMemsetAsync(red, 0, 2 * sizeof(unsigned long long), s));
-  const int ni = ix > 2 ? ix - 2 : 1, nj = jx > 2 ? jx - 2 : 1, nk = kx > 2 ? kx - 2 : 1;
-  const size_t total = (size_t)ni * nj * nk;
+  const unsigned groups = std::min(nblocks(speed_box(ix, jx, kx).count()), SPEED_GROUPS);
   if (ndim == 3)
-    k_speed<3><<<nblocks(total), TPB, 0, s>>>(a.dev, b.dev, ix, jx, kx, red, (int *)(red + 1));
+    k_speed<3><<<groups, TPB, 0, s>>>(a.dev, b.dev, ix, jx, kx, red, (int *)(red + 1));
   else
-    k_speed<2><<<nblocks(total), TPB, 0, s>>>(a.dev, b.dev, ix, jx, kx, red, (int *)(red + 1));
+    k_speed<2><<<groups, TPB, 0, s>>>(a.dev, b.dev, ix, jx, kx, red, (int *)(red + 1));
   OMHD_HIP(hipGetLastError());
   unsigned long long h[2];
   OMHD_HIP(hipMemcpyAsync(h, red, sizeof h, hipMemcpyDeviceToHost, s));
@@ -830,13 +862,9 @@ extern "C" int omhd_set_dt_noalloc(const double *U, const double *V, double *vma
   return ok();
 }
 
-static int bc_pair(double *dev, int ix, int jx, int kx, int dir, int tlo, int thi, const double *sl, const double *sh,
+static int bc_pair(double *dev, int ix, int jx, int kx, int dir, int tlo, const double *sl, const double *sh,
                    hipStream_t s) {
-  const int na = (dir == 1) ? jx : ix, nb = (dir == 3) ? jx : kx;
-  const size_t total = (size_t)na * nb;
-  k_bc_face_pair<<<nblocks(total), TPB, 0, s>>>(dev, ix, jx, kx, dir, tlo, thi, sl[0], sl[1], sl[2], sl[3], sl[4],
-                                                 sl[5], sl[6], sl[7], sl[8], sh[0], sh[1], sh[2], sh[3], sh[4], sh[5],
-                                                 sh[6], sh[7], sh[8]);
+  k_bc_face_pair<<<face_grid(ix, jx, kx, dir), TPB, 0, s>>>(dev, ix, jx, kx, dir, tlo, signs(sl, sh));
   OMHD_HIP(hipGetLastError());
   return OMHD_OK;
 }
@@ -855,11 +883,11 @@ extern "C" int omhd_bc_u(double *U, int32_t ix, int32_t jx, int32_t kx, const in
   Staged a;
   if (int rc = a.init(U, 9 * n, true, true, s)) return rc;
   if (ix > 2)
-    if (int rc = bc_pair(a.dev, ix, jx, kx, 1, bc_type[0], bc_type[1], sg, sg + 9, s)) return rc;
+    if (int rc = bc_pair(a.dev, ix, jx, kx, 1, bc_type[0], sg, sg + 9, s)) return rc;
   if (jx > 2)
-    if (int rc = bc_pair(a.dev, ix, jx, kx, 2, bc_type[2], bc_type[3], sg + 18, sg + 27, s)) return rc;
+    if (int rc = bc_pair(a.dev, ix, jx, kx, 2, bc_type[2], sg + 18, sg + 27, s)) return rc;
   if (kx > 2)
-    if (int rc = bc_pair(a.dev, ix, jx, kx, 3, bc_type[4], bc_type[5], sg + 36, sg + 45, s)) return rc;
+    if (int rc = bc_pair(a.dev, ix, jx, kx, 3, bc_type[4], sg + 36, sg + 45, s)) return rc;
   if (int rc = a.finish(s)) return rc;
   a.release(s);
   OMHD_HIP(hipStreamSynchronize(s));
@@ -878,12 +906,9 @@ extern "C" int omhd_bc_face(double *VL, double *VR, int32_t ix, int32_t jx, int3
   Staged l, r;
   if (int rc = l.init(VL, 9 * n, true, true, s)) return rc;
   if (int rc = r.init(VR, 9 * n, true, true, s)) return rc;
-  const int na = (dir == 1) ? jx : ix, nb = (dir == 3) ? jx : kx;
   const int nl = dir == 1 ? ix : dir == 2 ? jx : kx;
   if (nl >= 2) {
-    k_face_patch<<<nblocks((size_t)na * nb), TPB, 0, s>>>(l.dev, r.dev, ix, jx, kx, dir, bc_type, sl[0], sl[1], sl[2],
-                                                          sl[3], sl[4], sl[5], sl[6], sl[7], sl[8], sh[0], sh[1],
-                                                          sh[2], sh[3], sh[4], sh[5], sh[6], sh[7], sh[8]);
+    k_face_patch<<<face_grid(ix, jx, kx, dir), TPB, 0, s>>>(l.dev, r.dev, ix, jx, kx, dir, bc_type, signs(sl, sh));
     OMHD_HIP(hipGetLastError());
   }
   if (int rc = l.finish(s)) return rc;
