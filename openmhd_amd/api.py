@@ -61,7 +61,7 @@ def torch_ready(t) -> None:
         torch.cuda.current_stream(t.device).synchronize()
 
 
-def _ptr(a, n_expected: int | None = None):
+def _address(a, n_expected: int | None = None):
     """Device or host pointer of a float64 array laid out in Fortran order."""
     if a is None:
         return None
@@ -74,7 +74,6 @@ def _ptr(a, n_expected: int | None = None):
             raise ValueError("Fortran-ordered (column-major) contiguous tensor required")
         if n_expected is not None and a.numel() < n_expected:
             raise ValueError(f"tensor has {a.numel()} elements, expected {n_expected}")
-        torch_ready(a)
         return C.cast(C.c_void_p(a.data_ptr()), DP)
     if not isinstance(a, np.ndarray) or a.dtype != np.float64:
         raise TypeError("float64 numpy array required")
@@ -85,22 +84,42 @@ def _ptr(a, n_expected: int | None = None):
     return a.ctypes.data_as(DP)
 
 
+def _ptr(a, n_expected: int | None = None):
+    """_address of an array that torch's queued work has completed."""
+    p = _address(a, n_expected)
+    if hasattr(a, "data_ptr"):
+        torch_ready(a)
+    return p
+
+
+def _ptrs(*arrays):
+    """_ptr of each (array, elements expected), with one wait per device: it
+    covers every tensor of that device, and costs as much as a short kernel."""
+    ps = [_address(a, n) for a, n in arrays]
+    seen = []
+    for a, _ in arrays:
+        if hasattr(a, "data_ptr") and a.device not in seen:
+            seen.append(a.device)
+            torch_ready(a)
+    return ps
+
+
 def u2v(U, V, ix, jx, kx=1):
     """u2v(U,V,ix,jx) -- 2D_basic/u2v.f90:1 (3D: 3D_basic/u2v.f90:1)."""
     n = ix * jx * kx
-    check(lib.omhd_u2v(_ptr(U, 9 * n), _ptr(V, 4 * n), ix, jx, kx), "u2v")
+    check(lib.omhd_u2v(*_ptrs((U, 9 * n), (V, 4 * n)), ix, jx, kx), "u2v")
 
 
 def limiter(wk, wL, wR, ix, jx, dir, type, kx=1):
     """limiter(wk,wL,wR,ix,jx,dir,type) -- 2D_basic/limiter.f90:1."""
     n = ix * jx * kx
-    check(lib.omhd_limiter(_ptr(wk, n), _ptr(wL, n), _ptr(wR, n), ix, jx, kx, dir, type), "limiter")
+    check(lib.omhd_limiter(*_ptrs((wk, n), (wL, n), (wR, n)), ix, jx, kx, dir, type), "limiter")
 
 
 def flux_solver(F, VL, VR, ch, ix, jx, dir, type, kx=1):
     """flux_solver(F,VL,VR,ch,ix,jx,dir,type) -- 2D_basic/flux_solver.f90:1."""
     n = ix * jx * kx
-    check(lib.omhd_flux_solver(_ptr(F, 9 * n), _ptr(VL, 9 * n), _ptr(VR, 9 * n), ch, ix, jx, kx, dir, type),
+    check(lib.omhd_flux_solver(*_ptrs((F, 9 * n), (VL, 9 * n), (VR, 9 * n)), ch, ix, jx, kx, dir, type),
           "flux_solver")
 
 
@@ -111,7 +130,7 @@ def glm_ss2(U, ch, dt, ix, jx, kx=1):
 
 def _rk(mode, wk, wk1, wF, wG, dt, dx, ix, jx, wH, kx):
     n = 9 * ix * jx * kx
-    check(lib.omhd_rk(mode, _ptr(wk, n), _ptr(wk1, n), _ptr(wF, n), _ptr(wG, n), _ptr(wH, n), dt, dx, ix, jx, kx),
+    check(lib.omhd_rk(mode, *_ptrs((wk, n), (wk1, n), (wF, n), (wG, n), (wH, n)), dt, dx, ix, jx, kx),
           "rk")
 
 
@@ -140,7 +159,7 @@ def set_dt(U, V, dx, cfl, ix, jx, kx=1, ndim=2):
     Returns (vmax, dt), the reference's two output arguments."""
     vmax, dt = C.c_double(), C.c_double()
     n = ix * jx * kx
-    check(lib.omhd_set_dt(_ptr(U, 9 * n), _ptr(V, 4 * n), C.byref(vmax), C.byref(dt), dx, cfl, ix, jx, kx, ndim),
+    check(lib.omhd_set_dt(*_ptrs((U, 9 * n), (V, 4 * n)), C.byref(vmax), C.byref(dt), dx, cfl, ix, jx, kx, ndim),
           "set_dt")
     return vmax.value, dt.value
 
@@ -172,7 +191,7 @@ def _face(VL, VR, ix, jx, kx, dir, typ, slo, shi):
     n = 9 * ix * jx * kx
     a = np.ascontiguousarray(slo, dtype=np.float64)
     b = np.ascontiguousarray(shi, dtype=np.float64)
-    check(lib.omhd_bc_face(_ptr(VL, n), _ptr(VR, n), ix, jx, kx, dir, typ, a.ctypes.data_as(DP),
+    check(lib.omhd_bc_face(*_ptrs((VL, n), (VR, n)), ix, jx, kx, dir, typ, a.ctypes.data_as(DP),
                            b.ctypes.data_as(DP)), "bc_face")
 
 
@@ -262,7 +281,7 @@ def flux_resistive(F, U, x, y, dx, ix, jx, dir, eta=eta_recon):
     if len(x) != ix or len(y) != jx:
         raise ValueError(f"x, y have {len(x)}, {len(y)} points, expected {ix}, {jx}")
     t = eta_face_table(x, y, dx, dir, eta)
-    check(lib.omhd_flux_resistive(_ptr(F, 9 * n), _ptr(U, 9 * n), t.ctypes.data_as(DP), ix, jx, dir),
+    check(lib.omhd_flux_resistive(*_ptrs((F, 9 * n), (U, 9 * n)), t.ctypes.data_as(DP), ix, jx, dir),
           "flux_resistive")
 
 
@@ -278,7 +297,7 @@ def flux_resistive_3d(F, U, x, y, z, dx, ix, jx, kx, dir, eta=eta_recon):
     if len(x) != ix or len(y) != jx or len(z) != kx:
         raise ValueError(f"x, y, z have {len(x)}, {len(y)}, {len(z)} points, expected {ix}, {jx}, {kx}")
     t = eta_face_table(x, y, dx, dir, eta, over_dx=False)
-    check(lib.omhd_flux_resistive3d(_ptr(F, 9 * n), _ptr(U, 9 * n), t.ctypes.data_as(DP), 1, dx, ix, jx, kx, dir),
+    check(lib.omhd_flux_resistive3d(*_ptrs((F, 9 * n), (U, 9 * n)), t.ctypes.data_as(DP), 1, dx, ix, jx, kx, dir),
           "flux_resistive")
 
 

@@ -9,6 +9,7 @@
 #include <stdlib.h>
 
 #include <map>
+#include <condition_variable>
 #include <mutex>
 #include <vector>
 
@@ -130,15 +131,70 @@ hipStream_t dropin_stream() {
 }
 
 namespace {
+// What u2v and set_dt hand back besides arrays, without an allocation, a fill
+// and a copy per call (those and a second wait were 35 of the 50 us a call
+// took on 202^2 cells): `out`, two words of pinned host memory that the kernel
+// writes and the call reads after its one wait, and `red`, three device words
+// that every launch leaves zero.  CALL_SLOTS calls may be under way at once, in
+// any threads; a further one waits for a slot to be given back.
+constexpr int CALL_SLOTS = 64;
+struct CallSlot {
+  unsigned long long *out = nullptr, *red = nullptr;
+  int id = -1;
+  CallSlot() = default;
+  CallSlot(const CallSlot &) = delete;
+  CallSlot &operator=(const CallSlot &) = delete;
+  ~CallSlot() {
+    if (id < 0) return;
+    std::lock_guard<std::mutex> lock(pool().mu);
+    pool().free_ids.push_back(id);
+    pool().given_back.notify_one();
+  }
+  int acquire(hipStream_t s) {
+    Pool &p = pool();
+    std::unique_lock<std::mutex> lock(p.mu);
+    if (!p.red) {
+      unsigned long long *d = nullptr;
+      if (!p.out)
+        OMHD_HIP(hipHostMalloc((void **)&p.out, 2 * CALL_SLOTS * sizeof *p.out, hipHostMallocMapped | hipHostMallocCoherent));
+      OMHD_HIP(hipMallocAsync((void **)&d, 3 * CALL_SLOTS * sizeof *d, s));
+      OMHD_HIP(hipMemsetAsync(d, 0, 3 * CALL_SLOTS * sizeof *d, s));
+      OMHD_HIP(hipStreamSynchronize(s));
+      p.red = d;
+      for (int i = 0; i < CALL_SLOTS; i++) p.free_ids.push_back(i);
+    }
+    p.given_back.wait(lock, [&] { return !p.free_ids.empty(); });
+    id = p.free_ids.back();
+    p.free_ids.pop_back();
+    out = p.out + 2 * id;
+    red = p.red + 3 * id;
+    out[0] = out[1] = 0;
+    return OMHD_OK;
+  }
+
+ private:
+  struct Pool {
+    std::mutex mu;
+    std::condition_variable given_back;
+    std::vector<int> free_ids;
+    unsigned long long *out = nullptr, *red = nullptr;
+  };
+  static Pool &pool() {
+    static Pool *p = new Pool;  // outlives every thread that may still hold a slot
+    return *p;
+  }
+};
 
 constexpr int TPB = 256;
 
 inline unsigned nblocks(size_t n) { return (unsigned)((n + TPB - 1) / TPB); }
 
 // ---------------------------------------------------------------------------
-// u2v over all cells (u2v.f90:20-31); flags |= 1 for p <= 0, |= 2 for rho <= 0
+// u2v over all cells (u2v.f90:20-31); bad[0] = 1 if any p <= 0,
+// bad[1] = 1 if any rho <= 0 (host memory: one lane of a wavefront stores)
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_u2v(const double *__restrict__ U, double *__restrict__ V, size_t n, int *flags) {
+__global__ __launch_bounds__(256) void k_u2v(const double *__restrict__ U, double *__restrict__ V, size_t n,
+                                             unsigned long long *bad) {
   size_t c = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= n) return;
   double u[NV], w[NV];
@@ -147,10 +203,11 @@ __global__ __launch_bounds__(256) void k_u2v(const double *__restrict__ U, doubl
   cons_to_prim(u, w);
 #pragma unroll
   for (int m = 0; m < 4; m++) V[m * n + c] = w[m];
-  int f = 0;
-  if (w[3] <= 0) f |= 1;
-  if (u[4] <= 0) f |= 2;
-  if (f) atomicOr(flags, f);
+  const unsigned long long p_bad = __builtin_amdgcn_ballot_w64(w[3] <= 0), ro_bad = __builtin_amdgcn_ballot_w64(u[4] <= 0);
+  if ((p_bad | ro_bad) == 0) return;
+  const unsigned lane = threadIdx.x & 63;
+  if (p_bad && lane == (unsigned)__ffsll((long long)p_bad) - 1) bad[0] = 1;
+  if (ro_bad && lane == (unsigned)__ffsll((long long)ro_bad) - 1) bad[1] = 1;
 }
 
 // ---------------------------------------------------------------------------
@@ -317,7 +374,9 @@ __device__ __forceinline__ void group_reduce(double &v, int &f) {
 }
 
 // ---------------------------------------------------------------------------
-// set_dt: per-cell fastest speed, one atomic per workgroup.  SPEED_GROUPS
+// set_dt: per-cell fastest speed, one atomic per workgroup, max bits in red[0],
+// flags in red[1]; the workgroup that red[2] counts last hands them to out and
+// clears red for the next launch.  SPEED_GROUPS
 // workgroups at most, each over many cells: the atomics and the reads before
 // them all go to one address, so their number is bounded, and 2048 workgroups
 // fill the chip.  Bound by memory (64 B per cell).  160x128x120 cells: 40 us,
@@ -326,7 +385,7 @@ __device__ __forceinline__ void group_reduce(double &v, int &f) {
 constexpr unsigned SPEED_GROUPS = 2048;
 template <int ND>
 __global__ __launch_bounds__(256) void k_speed(const double *__restrict__ U, const double *__restrict__ V, int ix, int jx, int kx,
-                        unsigned long long *vmax_bits, int *flags) {
+                        unsigned long long *red, unsigned long long *out) {
   const Box b = speed_box(ix, jx, kx);
   const size_t total = b.count(), n = (size_t)ix * jx * kx, step = (size_t)gridDim.x * blockDim.x;
   double vt = 0.0;
@@ -341,8 +400,15 @@ __global__ __launch_bounds__(256) void k_speed(const double *__restrict__ U, con
   group_reduce(vt, f);
   if (threadIdx.x == 0) {
     if (f & 8) vt = __builtin_nan("");
-    if (f) atomicOr(flags, 4);
-    atomic_max_nonneg(vmax_bits, vt);
+    if (f) atomicOr(&red[1], 4ull);
+    atomic_max_nonneg(&red[0], vt);
+    __threadfence();
+    if (atomicAdd(&red[2], 1ull) == gridDim.x - 1) {  // the last workgroup
+      __threadfence();
+      out[0] = atomicExch(&red[0], 0ull);
+      out[1] = atomicExch(&red[1], 0ull);
+      atomicExch(&red[2], 0ull);
+    }
   }
 }
 
@@ -624,29 +690,24 @@ extern "C" int omhd_u2v(const double *U, double *V, int32_t ix, int32_t jx, int3
   hipStream_t s = dropin_stream();
   const size_t n = (size_t)ix * jx * kx;
   Staged dU, dV;
-  int *flags;
+  CallSlot slot;
   if (int rc = dU.init(U, 9 * n, true, false, s)) return rc;
   if (int rc = dV.init(V, 4 * n, false, true, s)) return rc;
-  OMHD_HIP(hipMallocAsync((void **)&flags, sizeof(int), s));
-  OMHD_HIP(hipMemsetAsync(flags, 0, sizeof(int), s));
-  k_u2v<<<nblocks(n), TPB, 0, s>>>(dU.dev, dV.dev, n, flags);
+  if (int rc = slot.acquire(s)) return rc;
+  k_u2v<<<nblocks(n), TPB, 0, s>>>(dU.dev, dV.dev, n, slot.out);
   OMHD_HIP(hipGetLastError());
-  int hflags = 0;
-  OMHD_HIP(hipMemcpyAsync(&hflags, flags, sizeof(int), hipMemcpyDeviceToHost, s));
   if (int rc = dV.finish(s)) return rc;
-  OMHD_HIP(hipStreamSynchronize(s));
-  (void)hipFreeAsync(flags, s);
   dU.release(s);
   dV.release(s);
   OMHD_HIP(hipStreamSynchronize(s));
-  if (hflags & 1) {  // u2v.f90:34-38: report minloc of p
+  if (slot.out[0]) {  // u2v.f90:34-38: report minloc of p
     double val;
     size_t c = plane_minloc(V + 3 * n, n, is_device_ptr(V), val);
     int i, j, k;
     unflatten(c, ix, jx, i, j, k);
     return set_error(OMHD_ERR_PRESSURE, "negative pressure", i, j, k, val);
   }
-  if (hflags & 2) {  // :39-43
+  if (slot.out[1]) {  // :39-43
     double val;
     size_t c = plane_minloc(U + 4 * n, n, is_device_ptr(U), val);
     int i, j, k;
@@ -787,21 +848,18 @@ extern "C" int omhd_set_dt(const double *U, const double *V, double *vmax, doubl
   Staged a, b;
   if (int rc = a.init(U, 9 * n, true, false, s)) return rc;
   if (int rc = b.init(V, 4 * n, true, false, s)) return rc;
-  unsigned long long *red;
-  OMHD_HIP(hipMallocAsync((void **)&red, 2 * sizeof(unsigned long long), s));
-  OMHD_HIP(hipMemsetAsync(red, 0, 2 * sizeof(unsigned long long), s));
+  CallSlot slot;
+  if (int rc = slot.acquire(s)) return rc;
   const unsigned groups = std::min(nblocks(speed_box(ix, jx, kx).count()), SPEED_GROUPS);
   if (ndim == 3)
-    k_speed<3><<<groups, TPB, 0, s>>>(a.dev, b.dev, ix, jx, kx, red, (int *)(red + 1));
+    k_speed<3><<<groups, TPB, 0, s>>>(a.dev, b.dev, ix, jx, kx, slot.red, slot.out);
   else
-    k_speed<2><<<groups, TPB, 0, s>>>(a.dev, b.dev, ix, jx, kx, red, (int *)(red + 1));
+    k_speed<2><<<groups, TPB, 0, s>>>(a.dev, b.dev, ix, jx, kx, slot.red, slot.out);
   OMHD_HIP(hipGetLastError());
-  unsigned long long h[2];
-  OMHD_HIP(hipMemcpyAsync(h, red, sizeof h, hipMemcpyDeviceToHost, s));
-  OMHD_HIP(hipStreamSynchronize(s));
-  (void)hipFreeAsync(red, s);
   a.release(s);
   b.release(s);
+  OMHD_HIP(hipStreamSynchronize(s));
+  const unsigned long long h[2] = {slot.out[0], slot.out[1]};
   double vm;
   memcpy(&vm, &h[0], sizeof vm);
   *vmax = vm;

@@ -75,3 +75,32 @@ def test_set_dt(oracle, shape):
     V[fast + (3,)] = np.nan  # the pressure: no speed of that cell is a number
     with pytest.raises(OMHDError):
         api.set_dt(U, V, 0.1, 0.4, *shape, nd)
+
+
+def test_calls_from_many_threads(oracle):
+    """u2v and set_dt share a bounded number of result slots: more threads than
+    slots, each with its own arrays, some with a cell that u2v reports."""
+    from concurrent.futures import ThreadPoolExecutor
+
+    from openmhd_amd import OMHDError, api
+
+    shape = (40, 30, 1)
+
+    def one(t):
+        rng = np.random.default_rng(t)
+        W = random_prim(rng, shape)
+        U, V, V2 = np.asfortranarray(prim_to_cons(W)), farr(*shape, 4), farr(*shape, 4)
+        oracle.u2v(U, V2)
+        want = oracle.set_dt(U, V2, 0.1, 0.4, 2)[1:]
+        bad = U.copy(order="F")
+        bad[t % 38 + 1, 3, 0, 3] = -5.0  # energy: a negative pressure
+        for _ in range(4):
+            api.u2v(U, V, *shape)
+            assert bits_equal(V, V2) and bits_equal(api.set_dt(U, V, 0.1, 0.4, *shape), want)
+            with pytest.raises(OMHDError) as e:
+                api.u2v(bad, V, *shape)
+            assert e.value.code == 1 and e.value.cell[0] == t % 38 + 2
+        return True
+
+    with ThreadPoolExecutor(80) as ex:
+        assert all(ex.map(one, range(80)))
