@@ -61,13 +61,26 @@ struct Geo {
   double dx;
 };
 
+// cell number t as its place i on row r (of ny * nz, fewer than 2^32): by a
+// 32-bit division where the grid allows (a 64-bit one is more instructions
+// than the smaller kernels here have)
+__device__ __forceinline__ void row_of(const Geo &g, unsigned long long t, int &i, unsigned &r) {
+  if ((unsigned long long)g.nx * g.ny * g.nz <= 0xffffffffull) {
+    r = (unsigned)t / (unsigned)g.nx;
+    i = (int)((unsigned)t - r * (unsigned)g.nx);
+  } else {
+    r = (unsigned)(t / (unsigned)g.nx);
+    i = (int)(t - (unsigned long long)r * (unsigned)g.nx);
+  }
+}
+
 __device__ __forceinline__ bool cell_of(const Geo &g, int &i, int &j, int &k) {
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (long long)g.nx * g.ny * g.nz) return false;
-  i = (int)(t % g.nx);
-  const long long r = t / g.nx;
-  j = (int)(r % g.ny);
-  k = (int)(r / g.ny);
+  const unsigned long long t = (unsigned long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= (unsigned long long)g.nx * g.ny * g.nz) return false;
+  unsigned r;
+  row_of(g, t, i, r);
+  k = (int)(r / (unsigned)g.ny);
+  j = (int)(r - (unsigned)k * (unsigned)g.ny);
   return true;
 }
 
@@ -81,16 +94,14 @@ __device__ __forceinline__ bool cell_of(const Geo &g, int &i, int &j, int &k) {
 __device__ __forceinline__ bool cell_of_tiled(const Geo &g, int &i, int &j, int &k) {
   const unsigned nb = gridDim.x, b = blockIdx.x;
   const unsigned L = (nb % 8u == 0u) ? (b % 8u) * (nb / 8u) + b / 8u : b;
-  const long long t = (long long)L * blockDim.x + threadIdx.x;
-  if (t >= (long long)g.nx * g.ny * g.nz) return false;
-  i = (int)(t % g.nx);
-  const long long q = t / g.nx;  // row ordinal in visiting order, < ny * nz
-  const int TY = min(16, g.ny & -g.ny), TZ = min(8, g.nz & -g.nz);
-  const int in = (int)(q % (TY * TZ));
-  const long long T = q / (TY * TZ);
-  const int nty = g.ny / TY;
-  j = (int)(T % nty) * TY + in % TY;
-  k = (int)(T / nty) * TZ + in / TY;
+  const unsigned long long t = (unsigned long long)L * blockDim.x + threadIdx.x;
+  if (t >= (unsigned long long)g.nx * g.ny * g.nz) return false;
+  unsigned q;  // row ordinal in visiting order, < ny * nz
+  row_of(g, t, i, q);
+  const unsigned TY = min(16, g.ny & -g.ny), TZ = min(8, g.nz & -g.nz);  // powers of two
+  const unsigned in = q & (TY * TZ - 1), T = q / (TY * TZ), nty = (unsigned)g.ny / TY, tz = T / nty;
+  j = (int)((T - tz * nty) * TY + (in & (TY - 1)));
+  k = (int)(tz * TZ + in / TY);
   return true;
 }
 
@@ -429,9 +440,10 @@ __global__ __launch_bounds__(256) void k_adj_res(const Geo g, const double *__re
   }
 }
 
-// res_gather for a cell one or more cells from every boundary: each role's
-// position is then read by exactly one face, (i,j,k) minus the role's shift,
-// with no ghost image; the same sums in the same order as res_gather.
+// res_gather for a cell one or more cells from every wall: each role's
+// position is then read by exactly one face, (i,j,k) minus the role's shift
+// (wrapped on a periodic axis), with no ghost image; the same sums in the same
+// order as res_gather.
 template <int DIR>
 __device__ __forceinline__ void res_gather_inner(const Geo &g, const double *__restrict__ F, int i, int j, int k,
                                                  double b[3]) {
@@ -441,7 +453,12 @@ __device__ __forceinline__ void res_gather_inner(const Geo &g, const double *__r
   constexpr int A1 = DIR == 0 ? 2 : (DIR == 1 ? 0 : 1);
   constexpr int A2 = DIR == 0 ? 1 : (DIR == 1 ? 2 : 0);
   const long long fp = fplane_of(g, DIR);
-  const int x[3] = {i, j, k};
+  const int x[3] = {i, j, k}, n[3] = {g.nx, g.ny, g.nz};
+  // x[a] - s: a wall face -1 of axis DIR is stored like the others, and a cell
+  // next to a wall does not come here, so only a periodic axis wraps
+  auto at = [&](int a, int s) {
+    return g.bc[a] == OMHD_BC_PERIODIC ? wrap_ax(x[a] - s, n[a]) : x[a] - s;
+  };
 #pragma unroll
   for (int dl = 0; dl < 2; dl++) {
 #pragma unroll
@@ -450,7 +467,7 @@ __device__ __forceinline__ void res_gather_inner(const Geo &g, const double *__r
       s[DIR] = dl;
       if (r == 1 || r == 2) s[A1] = r == 1 ? 1 : -1;
       if (r == 3 || r == 4) s[A2] = r == 3 ? 1 : -1;
-      const long long o = face_idx<DIR>(g, x[0] - s[0], x[1] - s[1], x[2] - s[2]);
+      const long long o = face_idx<DIR>(g, at(0, s[0]), at(1, s[1]), at(2, s[2]));
       if (r == 0) {
         const double bJ1 = F[o], bS1 = F[fp + o], bJ2 = F[2 * fp + o], bS2 = F[3 * fp + o];
         b[q1 - 5] += dl == 0 ? bJ1 + bS1 : -bJ1 + bS1;
@@ -467,13 +484,17 @@ __device__ __forceinline__ void res_gather_inner(const Geo &g, const double *__r
 }
 
 // second half: one thread per cell, the B adjoints from the faces of all
-// three axes, written to R (3 planes, slots bx, by, bz)
+// three axes, written to R (3 planes, slots bx, by, bz).  Bound by the loads (30
+// per cell, most of them from cache).  Only cells at a wall take the general
+// gather (82 us on 192x96x80 cells; 168 us when the ends of every periodic
+// row took it too, and two of three wavefronts with them).
 __global__ __launch_bounds__(256) void k_adj_res_gather(const Geo g, const double *__restrict__ rf,
                                                         double *__restrict__ R) {
   int i, j, k;
-  if (!cell_of(g, i, j, k)) return;
+  if (!cell_of_tiled(g, i, j, k)) return;
   double b[3] = {0.0, 0.0, 0.0};
-  if (i >= 1 && i <= g.nx - 2 && j >= 1 && j <= g.ny - 2 && k >= 1 && k <= g.nz - 2) {
+  auto inner = [&](int a, int c, int n) { return g.bc[a] == OMHD_BC_PERIODIC || (c >= 1 && c <= n - 2); };
+  if (inner(0, i, g.nx) && inner(1, j, g.ny) && inner(2, k, g.nz)) {
     res_gather_inner<0>(g, rf + fbase_of(g, 0), i, j, k, b);
     res_gather_inner<1>(g, rf + fbase_of(g, 1), i, j, k, b);
     res_gather_inner<2>(g, rf + fbase_of(g, 2), i, j, k, b);
@@ -488,7 +509,9 @@ __global__ __launch_bounds__(256) void k_adj_res_gather(const Geo g, const doubl
 }
 
 // the eta adjoints: one thread per entry (DIR, i+1, j+1) of geta, the face
-// (i, j) along DIR summed over k in increasing order and added to the entry
+// (i, j) along DIR summed over k in increasing order and added to the entry.
+// A chain of loads per thread, eight in flight (12 us on 192x96x80 cells, 38
+// one after the other).
 __global__ __launch_bounds__(256) void k_adj_eta(const Geo g, const double *__restrict__ rf,
                                                  double *__restrict__ geta) {
   const int ix = g.nx + 2, jx = g.ny + 2;
@@ -502,6 +525,7 @@ __global__ __launch_bounds__(256) void k_adj_eta(const Geo g, const double *__re
   const long long fp = fplane_of(g, d);
   const double *ge = rf + fbase_of(g, d) + 4 * fp;
   double s = 0.0;
+#pragma unroll 8
   for (int fk = (d == 2 && wz) ? -1 : 0; fk < g.nz; fk++)
     s += ge[((long long)(fk + (d == 2)) * fy + (fj + (d == 1))) * fx + (fi + (d == 0))];
   geta[t] += s;
