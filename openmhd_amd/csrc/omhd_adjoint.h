@@ -19,6 +19,10 @@
 #include <math.h>
 
 #if defined(__HIPCC__)
+#include "omhd_device.h"
+#endif
+
+#if defined(__HIPCC__)
 #define OMHD_HD __host__ __device__ inline
 #else
 #define OMHD_HD inline
@@ -350,103 +354,140 @@ OMHD_HD void hlld_fwd(const T L[NV], const T R[NV], double ch, T F[NV], int *bra
 }
 
 // ---------------------------------------------------------------------------
-// Reverse of one side's state block of hlld_fwd: given the adjoints of the
-// conserved momenta/energy U[0..3], of the physical flux FS, of the fast-mode
-// speed^2 a and of the total pressure pt, accumulate into bs (the side state).
+// Reverse of hlld_fwd.  Only the quantities its branches are decided by repeat
+// hlld_fwd's statements bit for bit; what only the reverse needs is left to
+// fused multiply-adds and plain reciprocals.
+//
+// Every side S enters the flux through FS - e US (its physical flux and e, the
+// fan speed where a star state follows it and 0 where it does not) and through
+// its star state.  The intermediate state Uh = iw (aR UR - aL UL - FR + FL)
+// has the same form, so with
+//   t_S[m] = [side S is taken] bF[m] +- iw bUh[m]        (+ for L, - for R)
+// one side function reverses (FS - e US) . t_S, the flux's and Uh's parts at
+// once, and the fan speeds get -US . t_S; no adjoints of FL, FR, UL and UR are
+// kept.  Uh and iw need no flux either: biw / iw = Uh . bUh.
 // ---------------------------------------------------------------------------
+#if defined(__clang__)
+#define OMHD_CONTRACT _Pragma("clang fp contract(fast)")
+#else
+#define OMHD_CONTRACT
+#endif
+
+// 1/x to an ulp
+OMHD_HD double rinv(double x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_amdgcn_div_fixup(recip(x), x, 1.0);
+#else
+  return 1.0 / x;
+#endif
+}
+// sqrt(x), correctly rounded
+OMHD_HD double root(double x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return csqrt(x);
+#else
+  return sqrt(x);
+#endif
+}
+
+// the side's quantities that hlld_fwd forms before the fans, and Uh's share
+// aS US - FS of its three momenta, density and transverse field
 template <int D>
-OMHD_HD void hlld_side_vjp(const double s[NV], const double bU[4], const double bFS[NV], double ba, double bpt,
-                           double bvB, double bs[NV]) {
+struct SideFwd {
+  double E, pt, vB, af;  // US[EN], total pressure, v.B, squared fast speed
+  double F[NV];          // FS[mn], [mt1], [mt2], [RO], [bt1], [bt2]
+};
+template <int D>
+OMHD_HD void side_fwd(const double S[NV], SideFwd<D> &o) {
   constexpr int vn = D, vt1 = (D + 1) % 3, vt2 = (D + 2) % 3;
-  constexpr int mn = vn, mt1 = vt1, mt2 = vt2;
+  constexpr int bn = 5 + vn, bt1 = 5 + vt1, bt2 = 5 + vt2;
+  constexpr int RO = 4, PR = 3;
+  const double r1 = 1.0 / (kGam - 1.0);
+  const double v2 = S[0] * S[0] + S[1] * S[1] + S[2] * S[2];
+  const double B2 = S[5] * S[5] + S[6] * S[6] + S[7] * S[7];
+  o.vB = S[0] * S[5] + S[1] * S[6] + S[2] * S[7];
+  o.E = 0.5 * (S[RO] * v2 + B2) + r1 * S[PR];
+  o.F[RO] = S[RO] * S[vn];
+  o.F[vn] = S[RO] * S[vn] * S[vn] - S[bn] * S[bn] + S[PR] + 0.5 * B2;
+  o.F[vt1] = S[RO] * S[vn] * S[vt1] - S[bn] * S[bt1];
+  o.F[vt2] = S[RO] * S[vn] * S[vt2] - S[bn] * S[bt2];
+  o.F[bt1] = S[vn] * S[bt1] - S[bn] * S[vt1];
+  o.F[bt2] = S[vn] * S[bt2] - S[bn] * S[vt2];
+  o.F[bn] = 0.0;
+  const double f1 = kGam * S[PR], f2 = 4 * (S[bn] * S[bn]);
+  o.af = ((f1 + B2) + root(tmax((f1 + B2) * (f1 + B2) - f1 * f2, 0.0))) / (2 * S[RO]);
+  o.pt = S[PR] + 0.5 * B2;
+}
+
+// bs += the reverse of (FS - e US) . t, of pt, vB and US[EN] with the adjoints
+// bpt, bvB and bE (e held), and of the squared fast speed af with ba
+template <int D>
+OMHD_HD void side_vjp(const double s[NV], const double t[NV], double e, double E, double pt, double vB, double af,
+                      double ba, double bpt, double bvB, double bE, double bs[NV]) {
+  OMHD_CONTRACT
+  constexpr int vn = D, vt1 = (D + 1) % 3, vt2 = (D + 2) % 3;
   constexpr int bn = 5 + vn, bt1 = 5 + vt1, bt2 = 5 + vt2;
   constexpr int RO = 4, PR = 3, EN = 3;
-  const double r1 = 1.0 / (kGam - 1.0), r2 = kGam / (kGam - 1.0);
-  const double ro = s[RO], p = s[PR];
-  const double v2 = s[0] * s[0] + s[1] * s[1] + s[2] * s[2];
-  const double B2 = s[5] * s[5] + s[6] * s[6] + s[7] * s[7];
-  const double vB = s[0] * s[5] + s[1] * s[6] + s[2] * s[7];
-  double bv2 = 0, bB2 = 0, bro = 0, bp = 0;
-  double bv[3] = {0, 0, 0}, bB[3] = {0, 0, 0};  // by velocity / field component index
-  // pt = p + 0.5 B2
-  bp += bpt;
-  bB2 += 0.5 * bpt;
-  // a = (A + sqrt(max(q, 0))) / (2 ro), A = f1 + B2, q = A*A - f1*f2
+  const double r1 = 1.0 / (kGam - 1.0);
+  // FS - e US, with c = vn - e: ro c (1, v) [density, momenta], mn: - bn^2 + pt,
+  // mt: - bn bt, bt: bt c - bn vt, en: E c + pt vn - bn vB
+  const double c = s[vn] - e, rc = s[RO] * c, tE = t[EN];
+  const double dot = s[0] * t[0] + s[1] * t[1] + s[2] * t[2] + t[RO];
+  const double bc = s[RO] * dot + E * tE + s[bt1] * t[bt1] + s[bt2] * t[bt2];
+  bE += c * tE;
+  bpt += t[vn] + s[vn] * tE;
+  bvB -= s[bn] * tE;
+  double bro = c * dot, bp = bpt + r1 * bE, bB2 = 0.5 * (bpt + bE);
+  double bv[3] = {0, 0, 0}, bB[3] = {0, 0, 0};
+  bv[vn] = bc + rc * t[vn] + pt * tE;
+  bv[vt1] = rc * t[vt1] - s[bn] * t[bt1];
+  bv[vt2] = rc * t[vt2] - s[bn] * t[bt2];
+  bB[vn] = -(2 * s[bn] * t[vn] + s[bt1] * t[vt1] + s[bt2] * t[vt2] + s[vt1] * t[bt1] + s[vt2] * t[bt2] + vB * tE);
+  bB[vt1] = c * t[bt1] - s[bn] * t[vt1];
+  bB[vt2] = c * t[bt2] - s[bn] * t[vt2];
+  // af = (A + sqrt(max(q, 0))) / (2 ro), A = f1 + B2, q = A*A - f1*f2
   {
-    const double f1 = kGam * p, f2 = 4 * (s[bn] * s[bn]);
-    const double A = f1 + B2;
+    const double B2 = s[5] * s[5] + s[6] * s[6] + s[7] * s[7];
+    const double f1 = kGam * s[PR], f2 = 4 * (s[bn] * s[bn]), A = f1 + B2;
     const double q = A * A - f1 * f2;
-    const double sq = sqrt(q > 0 ? q : 0.0);
-    const double ir = 1.0 / ro;  // reverse-only arithmetic: no correctly rounded quotients needed
-    const double a = (A + sq) * (0.5 * ir);
-    const double bN = 0.5 * ba * ir;
-    bro -= ba * a * ir;
-    double bA = bN;
-    const double bq = (q > 0 && sq > 0) ? bN / (2 * sq) : 0.0;
-    bA += 2 * A * bq;
-    double bf1 = -f2 * bq, bf2 = -f1 * bq;
-    bf1 += bA;
+    const double sq = root(q > 0 ? q : 0.0), ir = rinv(s[RO]), bN = 0.5 * ba * ir;
+    bro -= ba * af * ir;
+    const double bq = (q > 0 && sq > 0) ? bN * 0.5 * rinv(sq) : 0.0;
+    const double bA = bN + 2 * A * bq;
+    bp += kGam * (bA - f2 * bq);
     bB2 += bA;
-    bp += kGam * bf1;
-    bB[vn] += 8 * s[bn] * bf2;
+    bB[vn] -= 8 * s[bn] * (f1 * bq);
   }
-  // FS[bt2] = vn*bt2 - bn*vt2 ; FS[bt1]
-  bv[vn] += s[bt2] * bFS[bt2] + s[bt1] * bFS[bt1];
-  bB[vt2] += s[vn] * bFS[bt2];
-  bB[vn] -= s[vt2] * bFS[bt2] + s[vt1] * bFS[bt1];
-  bv[vt2] -= s[bn] * bFS[bt2];
-  bB[vt1] += s[vn] * bFS[bt1];
-  bv[vt1] -= s[bn] * bFS[bt1];
-  // FS[EN] = (0.5 ro v2 + r2 p + B2) vn - vB bn
-  {
-    const double E = 0.5 * ro * v2 + r2 * p + B2;
-    const double bE = s[vn] * bFS[EN];
-    bv[vn] += E * bFS[EN];
-    bvB -= s[bn] * bFS[EN];
-    bB[vn] -= vB * bFS[EN];
-    bro += 0.5 * v2 * bE;
-    bv2 += 0.5 * ro * bE;
-    bp += r2 * bE;
-    bB2 += bE;
-  }
-  // FS[mt] = ro vn vt - bn bt
-  bro += s[vn] * s[vt2] * bFS[mt2] + s[vn] * s[vt1] * bFS[mt1];
-  bv[vn] += ro * s[vt2] * bFS[mt2] + ro * s[vt1] * bFS[mt1];
-  bv[vt2] += ro * s[vn] * bFS[mt2];
-  bv[vt1] += ro * s[vn] * bFS[mt1];
-  bB[vn] -= s[bt2] * bFS[mt2] + s[bt1] * bFS[mt1];
-  bB[vt2] -= s[bn] * bFS[mt2];
-  bB[vt1] -= s[bn] * bFS[mt1];
-  // FS[mn] = ro vn vn - bn bn + p + 0.5 B2
-  bro += s[vn] * s[vn] * bFS[mn];
-  bv[vn] += 2 * ro * s[vn] * bFS[mn];
-  bB[vn] -= 2 * s[bn] * bFS[mn];
-  bp += bFS[mn];
-  bB2 += 0.5 * bFS[mn];
-  // FS[RO] = ro vn
-  bro += s[vn] * bFS[RO];
-  bv[vn] += ro * bFS[RO];
-  // U[EN] = 0.5 (ro v2 + B2) + r1 p ; U[m] = ro v_m
-  bro += 0.5 * v2 * bU[EN];
-  bv2 += 0.5 * ro * bU[EN];
-  bB2 += 0.5 * bU[EN];
-  bp += r1 * bU[EN];
-  for (int m = 0; m < 3; m++) {
-    bro += s[m] * bU[m];
-    bv[m] += ro * bU[m];
-  }
-  // vB, B2, v2
-  for (int m = 0; m < 3; m++) {
-    bv[m] += s[5 + m] * bvB + 2 * s[m] * bv2;
-    bB[m] += s[m] * bvB + 2 * s[5 + m] * bB2;
-  }
-  for (int m = 0; m < 3; m++) {
-    bs[m] += bv[m];
-    bs[5 + m] += bB[m];
-  }
+  // E = 0.5 (ro v2 + B2) + r1 p, pt = p + 0.5 B2, vB = v . B
+  const double v2 = s[0] * s[0] + s[1] * s[1] + s[2] * s[2], rE = s[RO] * bE;
+  bs[RO] += bro + 0.5 * v2 * bE;
   bs[PR] += bp;
-  bs[RO] += bro;
+  for (int m = 0; m < 3; m++) {
+    bs[m] += bv[m] + s[5 + m] * bvB + s[m] * rE;
+    bs[5 + m] += bB[m] + s[m] * bvB + 2 * s[5 + m] * bB2;
+  }
 }
+
+// the reverse of roS enS = Q / (aS - aM), the star energy of HLLD and HLLC-G:
+// Q = (aS - vn) E - ptS vn + pt aM + Uh[bn] P, P = vB - aM Uh[bn] - w1 c1 - w2 c2,
+// given bQ; w and c are the transverse velocity and field that P is formed with
+#define OMHD_STAR_ENERGY(S, aS, ES, ptS, enS, P, bQ, w1, w2, c1, c2, bw1, bw2, bc1, bc2, baS, bES, bptS, bvBS, bS) \
+  do {                                                                                                            \
+    const double bd_ = -(bQ) * (enS);                                                                             \
+    baS += bd_ + (ES) * (bQ);                                                                                     \
+    bS[vn] -= ((ES) + (ptS)) * (bQ);                                                                              \
+    bES += ((aS) - S[vn]) * (bQ);                                                                                 \
+    bptS -= S[vn] * (bQ);                                                                                         \
+    bpt += aM * (bQ);                                                                                             \
+    const double bP_ = Ubn * (bQ);                                                                                \
+    baM += pt * (bQ) - bd_ - Ubn * bP_;                                                                           \
+    bUh[bn] += (P) * (bQ)-aM * bP_;                                                                               \
+    bvBS += bP_;                                                                                                  \
+    bw1 -= (c1) * bP_;                                                                                            \
+    bc1 -= (w1) * bP_;                                                                                            \
+    bw2 -= (c2) * bP_;                                                                                            \
+    bc2 -= (w2) * bP_;                                                                                            \
+  } while (0)
 
 // bL += (dF/dL)^T bF, bR += (dF/dR)^T bF at the branch hlld_fwd takes.
 template <int D>
@@ -455,535 +496,259 @@ OMHD_HD void hlld_vjp(const double L[NV], const double R[NV], double ch, const d
   constexpr int vn = D, vt1 = (D + 1) % 3, vt2 = (D + 2) % 3;
   constexpr int mn = vn, mt1 = vt1, mt2 = vt2;
   constexpr int bn = 5 + vn, bt1 = 5 + vt1, bt2 = 5 + vt2;
-  constexpr int RO = 4, PR = 3, EN = 3, PS = 8;
-  const double r1 = 1.0 / (kGam - 1.0), r2 = kGam / (kGam - 1.0), hllg = 1.001;
-  // ---- forward recomputation (the same statements as hlld_fwd) ----
-  double UL[4], UR[4], FL[NV], FR[NV];
-  for (int m = 0; m < NV; m++) FL[m] = FR[m] = 0.0;
-  double v2 = L[0] * L[0] + L[1] * L[1] + L[2] * L[2];
-  double B2 = L[5] * L[5] + L[6] * L[6] + L[7] * L[7];
-  const double vBL = L[0] * L[5] + L[1] * L[6] + L[2] * L[7];
-  UL[0] = L[RO] * L[0];
-  UL[1] = L[RO] * L[1];
-  UL[2] = L[RO] * L[2];
-  UL[EN] = 0.5 * (L[RO] * v2 + B2) + r1 * L[PR];
-  FL[RO] = L[RO] * L[vn];
-  FL[mn] = L[RO] * L[vn] * L[vn] - L[bn] * L[bn] + L[PR] + 0.5 * B2;
-  FL[mt1] = L[RO] * L[vn] * L[vt1] - L[bn] * L[bt1];
-  FL[mt2] = L[RO] * L[vn] * L[vt2] - L[bn] * L[bt2];
-  FL[EN] = (0.5 * L[RO] * v2 + r2 * L[PR] + B2) * L[vn] - vBL * L[bn];
-  FL[bt1] = L[vn] * L[bt1] - L[bn] * L[vt1];
-  FL[bt2] = L[vn] * L[bt2] - L[bn] * L[vt2];
-  double f1 = kGam * L[PR];
-  double f2 = 4 * (L[bn] * L[bn]);
-  const double afL = ((f1 + B2) + sqrt(tmax((f1 + B2) * (f1 + B2) - f1 * f2, 0.0))) / (2 * L[RO]);
-  const double ptL = L[PR] + 0.5 * B2;
-  v2 = R[0] * R[0] + R[1] * R[1] + R[2] * R[2];
-  B2 = R[5] * R[5] + R[6] * R[6] + R[7] * R[7];
-  const double vBR = R[0] * R[5] + R[1] * R[6] + R[2] * R[7];
-  UR[0] = R[RO] * R[0];
-  UR[1] = R[RO] * R[1];
-  UR[2] = R[RO] * R[2];
-  UR[EN] = 0.5 * (R[RO] * v2 + B2) + r1 * R[PR];
-  FR[RO] = R[RO] * R[vn];
-  FR[mn] = R[RO] * R[vn] * R[vn] - R[bn] * R[bn] + R[PR] + 0.5 * B2;
-  FR[mt1] = R[RO] * R[vn] * R[vt1] - R[bn] * R[bt1];
-  FR[mt2] = R[RO] * R[vn] * R[vt2] - R[bn] * R[bt2];
-  FR[EN] = (0.5 * R[RO] * v2 + r2 * R[PR] + B2) * R[vn] - vBR * R[bn];
-  FR[bt1] = R[vn] * R[bt1] - R[bn] * R[vt1];
-  FR[bt2] = R[vn] * R[bt2] - R[bn] * R[vt2];
-  f1 = kGam * R[PR];
-  f2 = 4 * (R[bn] * R[bn]);
-  const double afR = ((f1 + B2) + sqrt(tmax((f1 + B2) * (f1 + B2) - f1 * f2, 0.0))) / (2 * R[RO]);
-  const double ptR = R[PR] + 0.5 * B2;
-  const double sa = sqrt(tmax(afL, afR));
-  const double aL = tmin(L[vn], R[vn]) - sa;
-  const double aR = tmax(L[vn], R[vn]) + sa;
-
-  // ---- adjoint accumulators ----
-  double bUL[4] = {0, 0, 0, 0}, bUR[4] = {0, 0, 0, 0};
-  double bFL[NV], bFR[NV];
-  for (int m = 0; m < NV; m++) bFL[m] = bFR[m] = 0.0;
-  double baL = 0, baR = 0;      // fan speeds SL, SR
-  double bptL = 0, bptR = 0, bvBL = 0, bvBR = 0;
-  // GLM pair (flux_solver.f90:580-581), every branch
-  bL[PS] += 0.5 * bF[bn] + 0.5 * ch * bF[PS];
-  bR[PS] += 0.5 * bF[bn] - 0.5 * ch * bF[PS];
-  bL[bn] += 0.5 * ch * bF[bn] + 0.5 * ch * ch * bF[PS];
-  bR[bn] += -0.5 * ch * bF[bn] + 0.5 * ch * ch * bF[PS];
-
-  if (aL >= 0) {
-    for (int m = 0; m < NV; m++)
-      if (m != bn && m != PS) bFL[m] += bF[m];
-  } else if (aR <= 0) {
-    for (int m = 0; m < NV; m++)
-      if (m != bn && m != PS) bFR[m] += bF[m];
-  } else {
-    double Uh[NV];
+  constexpr int RO = 4, EN = 3, PS = 8;
+  const double hllg = 1.001;
+  double EL, ER, ptL, ptR, vBL, vBR, afL, afR, sa, aL, aR;
+  double Uh[NV];  // slots mn, mt1, mt2, RO, bn, bt1, bt2
+  // the two sides' terms t, and the fan speed e of FS - e US
+  double tL[NV], tR[NV], eL = 0, eR = 0;
+  double baL = 0, baR = 0, bptL = 0, bptR = 0, bvBL = 0, bvBR = 0, bEL = 0, bER = 0;
+  {
+    SideFwd<D> l, r;
+    side_fwd<D>(L, l);
+    side_fwd<D>(R, r);
+    EL = l.E, ptL = l.pt, vBL = l.vB, afL = l.af;
+    ER = r.E, ptR = r.pt, vBR = r.vB, afR = r.af;
+    sa = root(tmax(afL, afR));
+    aL = tmin(L[vn], R[vn]) - sa;
+    aR = tmax(L[vn], R[vn]) + sa;
     const double iw = 1.0 / (aR - aL);
-    for (int m = 0; m < 3; m++) Uh[m] = iw * (aR * UR[m] - aL * UL[m] - FR[m] + FL[m]);
-    for (int m = RO; m <= 7; m++) Uh[m] = iw * (aR * R[m] - aL * L[m] - FR[m] + FL[m]);
-    Uh[3] = Uh[8] = 0.0;
+    for (int m = 0; m < 3; m++) Uh[m] = iw * (aR * (R[RO] * R[m]) - aL * (L[RO] * L[m]) - r.F[m] + l.F[m]);
+    for (int m = RO; m <= 7; m++) Uh[m] = iw * (aR * R[m] - aL * L[m] - r.F[m] + l.F[m]);
+  }
+  {  // GLM pair (flux_solver.f90:580-581), every branch
+    OMHD_CONTRACT
+    bL[PS] += 0.5 * bF[bn] + 0.5 * ch * bF[PS];
+    bR[PS] += 0.5 * bF[bn] - 0.5 * ch * bF[PS];
+    bL[bn] += 0.5 * ch * bF[bn] + 0.5 * ch * ch * bF[PS];
+    bR[bn] += -0.5 * ch * bF[bn] + 0.5 * ch * ch * bF[PS];
+  }
+  tL[bn] = tR[bn] = tL[PS] = tR[PS] = 0.0;
+  if (aL >= 0 || aR <= 0) {
+    const double kL = aL >= 0 ? 1.0 : 0.0, kR = aL >= 0 ? 0.0 : 1.0;
+    for (int m = 0; m < 8; m++)
+      if (m != bn) {
+        tL[m] = kL * bF[m];
+        tR[m] = kR * bF[m];
+      }
+  } else {
     const double aM = Uh[mn] / Uh[RO];
-    const double pt = ptL + L[RO] * (aL - L[vn]) * (aM - L[vn]);
     const double roL = L[RO] * (aL - L[vn]) / (aL - aM);
     const double roR = R[RO] * (aR - R[vn]) / (aR - aM);
-    const double hb = tabs(Uh[bn]);
-    const double sroL = sqrt(roL), sroR = sqrt(roR);
+    const double Ubn = Uh[bn], hb = tabs(Ubn);
+    const double sroL = root(roL), sroR = root(roR);
     const double aVL = hb / sroL;
     const double aVR = hb / sroR;
-    double bUh[NV];
-    for (int m = 0; m < NV; m++) bUh[m] = 0.0;
-    double biw = 0, baM = 0, bpt = 0, broL = 0, broR = 0, baVL = 0, baVR = 0;
-    if ((aL >= (aM - hllg * aVL)) || ((aM + hllg * aVR) >= aR)) {
+    const bool hllc = (aL >= (aM - hllg * aVL)) || ((aM + hllg * aVR) >= aR);
+    const double aL1 = aM - aVL;
+    const double aR1 = aM + aVR;
+    {
+    OMHD_CONTRACT
+    const double iw = rinv(aR - aL), iro = rinv(Uh[RO]), idL = rinv(aL - aM), idR = rinv(aR - aM);
+    const double dL = aL - L[vn], dR = aR - R[vn];
+    const double pt = ptL + L[RO] * dL * (aM - L[vn]);
+    double bUh[NV] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+    double baM = 0, bpt = 0, broL = 0, broR = 0;
+    eL = aL;
+    eR = aR;
+    tL[EN] = tR[EN] = 0.0;
+    if (hllc) {
       // ---- HLLC-G (flux_solver.f90:447-476) ----
-      const double w2 = aL * aR;
-      {
-        const double Nb1 = aR * FL[bt1] - aL * FR[bt1] + w2 * (R[bt1] - L[bt1]);
-        const double Nb2 = aR * FL[bt2] - aL * FR[bt2] + w2 * (R[bt2] - L[bt2]);
-        biw += Nb1 * bF[bt1] + Nb2 * bF[bt2];
-        const double b1 = iw * bF[bt1], b2 = iw * bF[bt2];
-        baR += FL[bt1] * b1 + FL[bt2] * b2;
-        bFL[bt1] += aR * b1;
-        bFL[bt2] += aR * b2;
-        baL -= FR[bt1] * b1 + FR[bt2] * b2;
-        bFR[bt1] -= aL * b1;
-        bFR[bt2] -= aL * b2;
-        const double bw2 = (R[bt1] - L[bt1]) * b1 + (R[bt2] - L[bt2]) * b2;
-        bR[bt1] += w2 * b1;
-        bL[bt1] -= w2 * b1;
-        bR[bt2] += w2 * b2;
-        bL[bt2] -= w2 * b2;
-        baL += aR * bw2;
-        baR += aL * bw2;
-      }
-      const double at1 = Uh[mt1] / Uh[RO];
-      const double at2 = Uh[mt2] / Uh[RO];
+      const double at1 = Uh[mt1] * iro, at2 = Uh[mt2] * iro;
       double bat1 = 0, bat2 = 0;
-      const bool useL = csign(0.5, aM) > 0;  // s1 = 0.5 + SIGN(0.5, aM) is 1 or 0
-      // the reverse of the side the flux takes, written once and inlined once
-      // per side, so every array it touches stays an ordinary register array
-      auto side = [&](const double *S, const double *US, double *bUS, double *bFS, double *bS, const double aS,
-                      const double roS, const double ptS, const double vBS, double &baS, double &broS,
+      auto side = [&](const double *S, double *bS, double *tS, const double aS, const double idS, const double roS,
+                      const double ES, const double ptS, const double vBS, double &baS, double &broS, double &bES,
                       double &bptS, double &bvBS) __attribute__((always_inline)) {
-        const double P = vBS - aM * Uh[bn] - at1 * Uh[bt1] - at2 * Uh[bt2];
-        const double Q = (aS - S[vn]) * US[EN] - ptS * S[vn] + pt * aM + Uh[bn] * P;
-        const double idS = 1.0 / (aS - aM);
-        const double enS = Q * idS;
-        // F[mn] = aS (roS aM - US[mn]) + FS[mn]
-        baS += (roS * aM - US[mn]) * bF[mn];
-        broS += aS * aM * bF[mn];
-        baM += aS * roS * bF[mn];
-        bUS[mn] -= aS * bF[mn];
-        bFS[mn] += bF[mn];
-        // F[mt1], F[mt2]
-        baS += (roS * at1 - US[mt1]) * bF[mt1] + (roS * at2 - US[mt2]) * bF[mt2];
-        broS += aS * at1 * bF[mt1] + aS * at2 * bF[mt2];
-        bat1 += aS * roS * bF[mt1];
-        bat2 += aS * roS * bF[mt2];
-        bUS[mt1] -= aS * bF[mt1];
-        bUS[mt2] -= aS * bF[mt2];
-        bFS[mt1] += bF[mt1];
-        bFS[mt2] += bF[mt2];
-        // F[EN] = aS (enS - US[EN]) + FS[EN]
-        baS += (enS - US[EN]) * bF[EN];
-        const double benS = aS * bF[EN];
-        bUS[EN] -= aS * bF[EN];
-        bFS[EN] += bF[EN];
-        // F[RO] = aS (roS - S[RO]) + FS[RO]
-        baS += (roS - S[RO]) * bF[RO];
-        broS += aS * bF[RO];
-        bS[RO] -= aS * bF[RO];
-        bFS[RO] += bF[RO];
-        // enS = Q / (aS - aM)
-        {
-          const double bQ = benS * idS;
-          const double bd = -bQ * enS;
-          baS += bd;
-          baM -= bd;
-          baS += US[EN] * bQ;
-          bS[vn] -= US[EN] * bQ + ptS * bQ;
-          bUS[EN] += (aS - S[vn]) * bQ;
-          bptS -= S[vn] * bQ;
-          bpt += aM * bQ;
-          baM += pt * bQ;
-          bUh[bn] += P * bQ;
-          const double bP = Uh[bn] * bQ;
-          bvBS += bP;
-          baM -= Uh[bn] * bP;
-          bUh[bn] -= aM * bP;
-          bat1 -= Uh[bt1] * bP;
-          bUh[bt1] -= at1 * bP;
-          bat2 -= Uh[bt2] * bP;
-          bUh[bt2] -= at2 * bP;
-        }
+        OMHD_CONTRACT
+        const double P = vBS - aM * Ubn - at1 * Uh[bt1] - at2 * Uh[bt2];
+        const double enS = ((aS - S[vn]) * ES - ptS * S[vn] + pt * aM + Ubn * P) * idS;
+        const double row = bF[RO] + aM * bF[mn] + at1 * bF[mt1] + at2 * bF[mt2];
+        const double x = aS * roS, bQ = aS * bF[EN] * idS;
+        tS[mn] = bF[mn];
+        tS[mt1] = bF[mt1];
+        tS[mt2] = bF[mt2];
+        tS[RO] = bF[RO];
+        tS[EN] = bF[EN];
+        baS += roS * row + enS * bF[EN];
+        broS += aS * row;
+        baM += x * bF[mn];
+        bat1 += x * bF[mt1];
+        bat2 += x * bF[mt2];
+        OMHD_STAR_ENERGY(S, aS, ES, ptS, enS, P, bQ, at1, at2, Uh[bt1], Uh[bt2], bat1, bat2, bUh[bt1], bUh[bt2], baS,
+                         bES, bptS, bvBS, bS);
       };
-      if (useL) side(L, UL, bUL, bFL, bL, aL, roL, ptL, vBL, baL, broL, bptL, bvBL);
-      else side(R, UR, bUR, bFR, bR, aR, roR, ptR, vBR, baR, broR, bptR, bvBR);
-      // at = Uh[mt] / Uh[RO]
-      const double iro = 1.0 / Uh[RO];
+      tL[mn] = tL[mt1] = tL[mt2] = tL[RO] = tR[mn] = tR[mt1] = tR[mt2] = tR[RO] = 0.0;
+      // s1 = 0.5 + SIGN(0.5, aM) is 1 (left) or 0
+      if (csign(0.5, aM) > 0) side(L, bL, tL, aL, idL, roL, EL, ptL, vBL, baL, broL, bEL, bptL, bvBL);
+      else side(R, bR, tR, aR, idR, roR, ER, ptR, vBR, baR, broR, bER, bptR, bvBR);
       bUh[mt1] += bat1 * iro;
       bUh[mt2] += bat2 * iro;
       bUh[RO] -= (at1 * bat1 + at2 * bat2) * iro;
+      // F[bt] = iw (aR FL - aL FR + aL aR (R - L)): FL - aL L with the factor iw aR, FR - aR R with -iw aL
+      double g = 0;
+      for (int q = 0; q < 2; q++) {
+        const int bt = q ? bt2 : bt1, vt = q ? vt2 : vt1;
+        const double be = iw * bF[bt];
+        const double fl = L[vn] * L[bt] - L[bn] * L[vt], fr = R[vn] * R[bt] - R[bn] * R[vt];
+        tL[bt] = aR * be;
+        tR[bt] = -aL * be;
+        baL += (aR * R[bt] - fr) * be;
+        baR += (fl - aL * L[bt]) * be;
+        g += iw * (aR * fl - aL * fr + aL * aR * (R[bt] - L[bt])) * be;
+      }
+      baR -= g;
+      baL += g;
     } else {
       // ---- HLLD (flux_solver.f90:482-572) ----
-      double UL1[NV], UR1[NV];
-      const double dL = L[RO] * (aL - L[vn]) * (aL - aM) - Uh[bn] * Uh[bn];
-      const double f1L = 1.0 / dL;
-      const double eL = L[RO] * ((aL - L[vn]) * (aL - L[vn])) - Uh[bn] * Uh[bn];
-      UL1[bt1] = L[bt1] * f1L * eL;
-      UL1[bt2] = L[bt2] * f1L * eL;
-      const double vt1L = L[vt1] - f1L * Uh[bn] * L[bt1] * (aM - L[vn]);
-      const double vt2L = L[vt2] - f1L * Uh[bn] * L[bt2] * (aM - L[vn]);
-      UL1[RO] = roL;
-      const double PL = vBL - aM * Uh[bn] - vt1L * UL1[bt1] - vt2L * UL1[bt2];
-      const double QL = (aL - L[vn]) * UL[EN] - ptL * L[vn] + pt * aM + Uh[bn] * PL;
-      UL1[EN] = QL / (aL - aM);
-      UL1[mn] = roL * aM;
-      UL1[mt1] = roL * vt1L;
-      UL1[mt2] = roL * vt2L;
-      const double dR = R[RO] * (aR - R[vn]) * (aR - aM) - Uh[bn] * Uh[bn];
-      const double f1R = 1.0 / dR;
-      const double eR = R[RO] * ((aR - R[vn]) * (aR - R[vn])) - Uh[bn] * Uh[bn];
-      UR1[bt1] = R[bt1] * f1R * eR;
-      UR1[bt2] = R[bt2] * f1R * eR;
-      const double vt1R = R[vt1] - f1R * Uh[bn] * R[bt1] * (aM - R[vn]);
-      const double vt2R = R[vt2] - f1R * Uh[bn] * R[bt2] * (aM - R[vn]);
-      UR1[RO] = roR;
-      const double PR_ = vBR - aM * Uh[bn] - vt1R * UR1[bt1] - vt2R * UR1[bt2];
-      const double QR = (aR - R[vn]) * UR[EN] - ptR * R[vn] + pt * aM + Uh[bn] * PR_;
-      UR1[EN] = QR / (aR - aM);
-      UR1[mn] = roR * aM;
-      UR1[mt1] = roR * vt1R;
-      UR1[mt2] = roR * vt2R;
-      const double aL1 = aM - aVL;
-      const double aR1 = aM + aVR;
-      double bUL1[NV], bUR1[NV];
-      for (int m = 0; m < NV; m++) bUL1[m] = bUR1[m] = 0.0;
-      double bvt1L = 0, bvt2L = 0, bvt1R = 0, bvt2R = 0, baL1 = 0, baR1 = 0;
-      // indices of the flux slots a star-state branch writes: momenta + EN
-      // (cons slots 0..3), RO, bt1, bt2
-      if (aL1 >= 0) {
-        for (int m = 0; m < 4; m++) {
-          baL += (UL1[m] - UL[m]) * bF[m];
-          bUL1[m] += aL * bF[m];
-          bUL[m] -= aL * bF[m];
-          bFL[m] += bF[m];
-        }
-        for (int q = 0; q < 3; q++) {
-          const int m = q == 0 ? RO : (q == 1 ? bt1 : bt2);
-          baL += (UL1[m] - L[m]) * bF[m];
-          bUL1[m] += aL * bF[m];
-          bL[m] -= aL * bF[m];
-          bFL[m] += bF[m];
-        }
-      } else if (aR1 <= 0) {
-        for (int m = 0; m < 4; m++) {
-          baR += (UR1[m] - UR[m]) * bF[m];
-          bUR1[m] += aR * bF[m];
-          bUR[m] -= aR * bF[m];
-          bFR[m] += bF[m];
-        }
-        for (int q = 0; q < 3; q++) {
-          const int m = q == 0 ? RO : (q == 1 ? bt1 : bt2);
-          baR += (UR1[m] - R[m]) * bF[m];
-          bUR1[m] += aR * bF[m];
-          bR[m] -= aR * bF[m];
-          bFR[m] += bF[m];
-        }
-      } else {
-        // central states (flux_solver.f90:533-572)
-        double U2[NV], bU2[NV];
-        for (int m = 0; m < NV; m++) bU2[m] = 0.0;
-        const double roLs = sroL, roRs = sroR;
-        const double fc = 1.0 / (roLs + roRs);
-        const double sB = csign(1.0, Uh[bn]);
-        const double Na1 = roLs * vt1L + roRs * vt1R + (UR1[bt1] - UL1[bt1]) * sB;
-        const double Na2 = roLs * vt2L + roRs * vt2R + (UR1[bt2] - UL1[bt2]) * sB;
-        const double at1 = fc * Na1, at2 = fc * Na2;
-        const double Nb1 = roLs * UR1[bt1] + roRs * UL1[bt1] + roLs * roRs * (vt1R - vt1L) * sB;
-        const double Nb2 = roLs * UR1[bt2] + roRs * UL1[bt2] + roLs * roRs * (vt2R - vt2L) * sB;
-        U2[bt1] = fc * Nb1;
-        U2[bt2] = fc * Nb2;
-        double broLs = 0, broRs = 0, bat1 = 0, bat2 = 0;
-        const bool left = aM >= 0;
-        // the side whose double-star state the flux takes (L** or R**), inlined
-        // once per side so every array it touches stays a register array
-        auto central_side = [&](const double *S, const double *US, const double *US1, double *bUS, double *bUS1,
-                                double *bFS, double *bS, const double aS, const double aS1, const double roS,
-                                const double roSs, const double vt1S, const double vt2S, const double sgn,
-                                double &baS, double &baS1, double &broS, double &broSs, double &bvt1S,
-                                double &bvt2S) __attribute__((always_inline)) {
-          U2[RO] = roS;
-          const double K = vt1S * US1[bt1] + vt2S * US1[bt2] - at1 * U2[bt1] - at2 * U2[bt2];
-          U2[EN] = US1[EN] + sgn * roSs * K * sB;
-          U2[mn] = roS * aM;
-          U2[mt1] = roS * at1;
-          U2[mt2] = roS * at2;
-          // F[m] = aS1 U2[m] - (aS1 - aS) US1[m] - aS XS[m] + FS[m]
-          for (int m = 0; m < 4; m++) {
-            baS1 += (U2[m] - US1[m]) * bF[m];
-            bU2[m] += aS1 * bF[m];
-            bUS1[m] -= (aS1 - aS) * bF[m];
-            baS += (US1[m] - US[m]) * bF[m];
-            bUS[m] -= aS * bF[m];
-            bFS[m] += bF[m];
-          }
-          for (int q = 0; q < 3; q++) {
-            const int m = q == 0 ? RO : (q == 1 ? bt1 : bt2);
-            baS1 += (U2[m] - US1[m]) * bF[m];
-            bU2[m] += aS1 * bF[m];
-            bUS1[m] -= (aS1 - aS) * bF[m];
-            baS += (US1[m] - S[m]) * bF[m];
-            bS[m] -= aS * bF[m];
-            bFS[m] += bF[m];
-          }
-          // U2[mt] = roS at, U2[mn] = roS aM, U2[RO] = roS
-          broS += at2 * bU2[mt2] + at1 * bU2[mt1] + aM * bU2[mn] + bU2[RO];
-          bat2 += roS * bU2[mt2];
-          bat1 += roS * bU2[mt1];
-          baM += roS * bU2[mn];
-          // U2[EN] = US1[EN] + sgn roSs K sB
-          {
-            const double b = bU2[EN];
-            bUS1[EN] += b;
-            broSs += sgn * K * sB * b;
-            const double bK = sgn * roSs * sB * b;
-            bvt1S += US1[bt1] * bK;
-            bUS1[bt1] += vt1S * bK;
-            bvt2S += US1[bt2] * bK;
-            bUS1[bt2] += vt2S * bK;
-            bat1 -= U2[bt1] * bK;
-            bU2[bt1] -= at1 * bK;
-            bat2 -= U2[bt2] * bK;
-            bU2[bt2] -= at2 * bK;
-          }
-        };
-        // sgn: L** is UL1[EN] - roLs(...)sB, R** is UR1[EN] + roRs(...)sB
-        if (left)
-          central_side(L, UL, UL1, bUL, bUL1, bFL, bL, aL, aL1, roL, roLs, vt1L, vt2L, -1.0, baL, baL1, broL, broLs,
-                       bvt1L, bvt2L);
-        else
-          central_side(R, UR, UR1, bUR, bUR1, bFR, bR, aR, aR1, roR, roRs, vt1R, vt2R, 1.0, baR, baR1, broR, broRs,
-                       bvt1R, bvt2R);
-        double bfc = 0;
-        // U2[bt] = fc * Nb
-        {
-          bfc += Nb1 * bU2[bt1] + Nb2 * bU2[bt2];
-          const double n1 = fc * bU2[bt1], n2 = fc * bU2[bt2];
-          broLs += UR1[bt1] * n1 + UR1[bt2] * n2;
-          bUR1[bt1] += roLs * n1;
-          bUR1[bt2] += roLs * n2;
-          broRs += UL1[bt1] * n1 + UL1[bt2] * n2;
-          bUL1[bt1] += roRs * n1;
-          bUL1[bt2] += roRs * n2;
-          const double bP = (vt1R - vt1L) * sB * n1 + (vt2R - vt2L) * sB * n2;
-          const double P = roLs * roRs;
-          bvt1R += P * sB * n1;
-          bvt1L -= P * sB * n1;
-          bvt2R += P * sB * n2;
-          bvt2L -= P * sB * n2;
-          broLs += roRs * bP;
-          broRs += roLs * bP;
-        }
-        // at = fc * Na
-        {
-          bfc += Na1 * bat1 + Na2 * bat2;
-          const double n1 = fc * bat1, n2 = fc * bat2;
-          broLs += vt1L * n1 + vt2L * n2;
-          bvt1L += roLs * n1;
-          bvt2L += roLs * n2;
-          broRs += vt1R * n1 + vt2R * n2;
-          bvt1R += roRs * n1;
-          bvt2R += roRs * n2;
-          bUR1[bt1] += sB * n1;
-          bUL1[bt1] -= sB * n1;
-          bUR1[bt2] += sB * n2;
-          bUL1[bt2] -= sB * n2;
-        }
-        // fc = 1 / (roLs + roRs); roXs = sqrt(roX)
-        {
-          const double bs = -fc * fc * bfc;
-          broLs += bs;
-          broRs += bs;
-          broL += broLs * 0.5 * sroL / roL;  // d sqrt(ro) = d ro / (2 sqrt(ro))
-          broR += broRs * 0.5 * sroR / roR;
-        }
+      const double f1L = rinv(L[RO] * dL * (aL - aM) - Ubn * Ubn), f1R = rinv(R[RO] * dR * (aR - aM) - Ubn * Ubn);
+      const double gL = f1L * (L[RO] * dL * dL - Ubn * Ubn), gR = f1R * (R[RO] * dR * dR - Ubn * Ubn);
+      const double b1L = L[bt1] * gL, b2L = L[bt2] * gL, b1R = R[bt1] * gR, b2R = R[bt2] * gR;
+      const double hL = f1L * Ubn * (aM - L[vn]), hR = f1R * Ubn * (aM - R[vn]);
+      const double v1L = L[vt1] - hL * L[bt1], v2L = L[vt2] - hL * L[bt2];
+      const double v1R = R[vt1] - hR * R[bt1], v2R = R[vt2] - hR * R[bt2];
+      const bool central = aL1 < 0 && aR1 > 0;
+      const bool left = central ? aM >= 0 : aL1 >= 0;
+      const double kL = left ? 1.0 : 0.0, kR = left ? 0.0 : 1.0;
+      const double isL = rinv(sroL), isR = rinv(sroR);
+      double bv1L = 0, bv2L = 0, bv1R = 0, bv2R = 0, bb1L = 0, bb2L = 0, bb1R = 0, bb2R = 0;
+      double bsL = 0, bsR = 0, ba1L = 0, ba1R = 0;  // sqrt(roS), aL1 and aR1
+      if (central) {  // central states (flux_solver.f90:533-572)
+        const double sB = csign(1.0, Ubn), fc = rinv(sroL + sroR), P = sroL * sroR * sB;
+        const double at1 = fc * (sroL * v1L + sroR * v1R + (b1R - b1L) * sB);
+        const double at2 = fc * (sroL * v2L + sroR * v2R + (b2R - b2L) * sB);
+        const double B1 = fc * (sroL * b1R + sroR * b1L + P * (v1R - v1L));
+        const double B2 = fc * (sroL * b2R + sroR * b2L + P * (v2R - v2L));
+        // the side taken: U2 = (roT, roT aM, roT at, UT1[EN] + sT K, B)
+        const double w = left ? aL1 : aR1, roT = left ? roL : roR, sT = left ? -sroL * sB : sroR * sB;
+        const double v1T = left ? v1L : v1R, v2T = left ? v2L : v2R, b1T = left ? b1L : b1R, b2T = left ? b2L : b2R;
+        const double K = v1T * b1T + v2T * b2T - at1 * B1 - at2 * B2;
+        const double bK = w * bF[EN] * sT, wr = w * roT, bs = K * sB * w * bF[EN];
+        const double ba1 = roT * ((at1 - v1T) * bF[mt1] + (at2 - v2T) * bF[mt2]) + sT * K * bF[EN] +
+                           (B1 - b1T) * bF[bt1] + (B2 - b2T) * bF[bt2];
+        const double bro = w * (at1 * bF[mt1] + at2 * bF[mt2]);
+        ba1L = kL * ba1;
+        ba1R = kR * ba1;
+        broL += kL * bro;
+        broR += kR * bro;
+        // fc (at), fc (B) reversed: a = fc bat, n = fc bB
+        const double a1 = fc * (wr * bF[mt1] - B1 * bK), a2 = fc * (wr * bF[mt2] - B2 * bK);
+        const double n1 = fc * (w * bF[bt1] - at1 * bK), n2 = fc * (w * bF[bt2] - at2 * bK);
+        const double z = at1 * a1 + at2 * a2 + B1 * n1 + B2 * n2;  // the adjoint of fc times -fc
+        const double bP = ((v1R - v1L) * n1 + (v2R - v2L) * n2) * sB;
+        bsL = b1R * n1 + b2R * n2 + v1L * a1 + v2L * a2 + sroR * bP - z - kL * bs;
+        bsR = b1L * n1 + b2L * n2 + v1R * a1 + v2R * a2 + sroL * bP - z + kR * bs;
+        const double KL = kL * bK, KR = kR * bK;
+        bv1L = sroL * a1 - P * n1 + KL * b1L;
+        bv2L = sroL * a2 - P * n2 + KL * b2L;
+        bv1R = sroR * a1 + P * n1 + KR * b1R;
+        bv2R = sroR * a2 + P * n2 + KR * b2R;
+        bb1L = sroR * n1 - sB * a1 + KL * v1L;
+        bb2L = sroR * n2 - sB * a2 + KL * v2L;
+        bb1R = sroL * n1 + sB * a1 + KR * v1R;
+        bb2R = sroL * n2 + sB * a2 + KR * v2R;
       }
-      // aL1 = aM - aVL, aR1 = aM + aVR
-      baM += baL1 + baR1;
-      baVL -= baL1;
-      baVR += baR1;
-      // star states, right then left (statements of flux_solver.f90:482-507)
-      for (int side = 1; side >= 0; side--) {
-        const bool Ls = side == 0;
-        const double *S = Ls ? L : R;
-        const double *US = Ls ? UL : UR;
-        const double *US1 = Ls ? UL1 : UR1;
-        double *bUS1 = Ls ? bUL1 : bUR1;
-        double *bUS = Ls ? bUL : bUR;
-        double *bS = Ls ? bL : bR;
-        const double aS = Ls ? aL : aR;
-        const double roS = Ls ? roL : roR;
-        const double ptS = Ls ? ptL : ptR;
-        const double f1S = Ls ? f1L : f1R;
-        const double eS = Ls ? eL : eR;
-        const double PS_ = Ls ? PL : PR_;
-        const double vt1S = Ls ? vt1L : vt1R, vt2S = Ls ? vt2L : vt2R;
-        double &baS = Ls ? baL : baR;
-        double &broS = Ls ? broL : broR;
-        double &bptS = Ls ? bptL : bptR;
-        double &bvBS = Ls ? bvBL : bvBR;
-        double bvt1S = Ls ? bvt1L : bvt1R, bvt2S = Ls ? bvt2L : bvt2R;
-        // US1[mt] = roS vtS, US1[mn] = roS aM, US1[RO] = roS
-        broS += vt2S * bUS1[mt2] + vt1S * bUS1[mt1] + aM * bUS1[mn] + bUS1[RO];
-        bvt2S += roS * bUS1[mt2];
-        bvt1S += roS * bUS1[mt1];
-        baM += roS * bUS1[mn];
-        // US1[EN] = QS / (aS - aM)
-        {
-          const double bQ = bUS1[EN] / (aS - aM);
-          const double bd = -bQ * US1[EN];
-          baS += bd;
-          baM -= bd;
-          baS += US[EN] * bQ;
-          bS[vn] -= US[EN] * bQ + ptS * bQ;
-          bUS[EN] += (aS - S[vn]) * bQ;
-          bptS -= S[vn] * bQ;
-          bpt += aM * bQ;
-          baM += pt * bQ;
-          bUh[bn] += PS_ * bQ;
-          const double bP = Uh[bn] * bQ;
-          bvBS += bP;
-          baM -= Uh[bn] * bP;
-          bUh[bn] -= aM * bP;
-          bvt1S -= US1[bt1] * bP;
-          bUS1[bt1] -= vt1S * bP;
-          bvt2S -= US1[bt2] * bP;
-          bUS1[bt2] -= vt2S * bP;
-        }
-        double bf1S = 0, beS = 0;
-        // vtS = S[vt] - f1S Uh[bn] S[bt] (aM - S[vn])
-        for (int t = 0; t < 2; t++) {
-          const int vt = t ? vt2 : vt1, bt = t ? bt2 : bt1;
-          const double b = t ? bvt2S : bvt1S;
-          const double G = f1S * Uh[bn] * S[bt];
-          bS[vt] += b;
-          const double bG = -(aM - S[vn]) * b;
-          baM -= G * b;
-          bS[vn] += G * b;
-          bf1S += Uh[bn] * S[bt] * bG;
-          bUh[bn] += f1S * S[bt] * bG;
-          bS[bt] += f1S * Uh[bn] * bG;
-        }
-        // US1[bt] = S[bt] f1S eS
-        for (int t = 0; t < 2; t++) {
-          const int bt = t ? bt2 : bt1;
-          bS[bt] += f1S * eS * bUS1[bt];
-          bf1S += S[bt] * eS * bUS1[bt];
-          beS += S[bt] * f1S * bUS1[bt];
-        }
-        // eS = S[RO] (aS - S[vn])^2 - Uh[bn]^2
-        {
-          const double dd = aS - S[vn];
-          bS[RO] += dd * dd * beS;
-          const double bdd = 2 * S[RO] * dd * beS;
-          baS += bdd;
-          bS[vn] -= bdd;
-          bUh[bn] -= 2 * Uh[bn] * beS;
-        }
-        // f1S = 1 / dS, dS = S[RO] (aS - S[vn]) (aS - aM) - Uh[bn]^2
-        {
-          const double bd = -f1S * f1S * bf1S;
-          const double p1 = aS - S[vn], p2 = aS - aM;
-          bS[RO] += p1 * p2 * bd;
-          baS += S[RO] * p2 * bd + S[RO] * p1 * bd;
-          bS[vn] -= S[RO] * p2 * bd;
-          baM -= S[RO] * p1 * bd;
-          bUh[bn] -= 2 * Uh[bn] * bd;
-        }
-      }
+      // aL1 = aM - aVL, aR1 = aM + aVR, aVS = |Uh[bn]| / sqrt(roS)
+      baM += ba1L + ba1R;
+      bUh[bn] += (Ubn < 0 ? -1.0 : 1.0) * (ba1R * isR - ba1L * isL);
+      broL += 0.5 * isL * (bsL + ba1L * aVL * isL);
+      broR += 0.5 * isR * (bsR - ba1R * aVR * isR);
+      // the star states, reversed side by side
+      auto star = [&](const double *S, double *bS, double *tS, const double k, const double aS, const double y,
+                      const double dS, const double idS, const double roS, const double ES, const double ptS,
+                      const double vBS, const double f1, const double g, const double v1, const double v2,
+                      const double b1, const double b2, double bv1, double bv2, double bb1, double bb2, double &baS,
+                      double &broS, double &bES, double &bptS, double &bvBS) __attribute__((always_inline)) {
+        OMHD_CONTRACT
+        // F takes aS US1 (S*), or (aS - aS1) US1 + aS1 U2 (S**): y is the factor of US1's transverse parts
+        const double P = vBS - aM * Ubn - v1 * b1 - v2 * b2;
+        const double en = (dS * ES - ptS * S[vn] + pt * aM + Ubn * P) * idS;
+        const double x = k * aS, row = bF[RO] + aM * bF[mn], rot = v1 * bF[mt1] + v2 * bF[mt2];
+        for (int m = 0; m < 8; m++)
+          if (m != bn) tS[m] = k * bF[m];
+        baS += k * (roS * (row + rot) + en * bF[EN] + b1 * bF[bt1] + b2 * bF[bt2]);
+        broS += x * row + y * rot;
+        baM += x * roS * bF[mn];
+        bv1 += y * roS * bF[mt1];
+        bv2 += y * roS * bF[mt2];
+        bb1 += y * bF[bt1];
+        bb2 += y * bF[bt2];
+        const double bQ = x * bF[EN] * idS;
+        OMHD_STAR_ENERGY(S, aS, ES, ptS, en, P, bQ, v1, v2, b1, b2, bv1, bv2, bb1, bb2, baS, bES, bptS, bvBS, bS);
+        // v = S[vt] - f1 Uh[bn] S[bt] (aM - vn), b = S[bt] f1 e, e = ro (aS - vn)^2 - Uh[bn]^2,
+        // 1/f1 = ro (aS - vn) (aS - aM) - Uh[bn]^2
+        const double c = aM - S[vn], fU = f1 * Ubn;
+        const double sv = S[bt1] * bv1 + S[bt2] * bv2, sb = S[bt1] * bb1 + S[bt2] * bb2;
+        bS[vt1] += bv1;
+        bS[vt2] += bv2;
+        bS[bt1] += g * bb1 - fU * c * bv1;
+        bS[bt2] += g * bb2 - fU * c * bv2;
+        const double be = f1 * sb, bd = -f1 * (g * sb - fU * c * sv), p2 = aS - aM, rd = S[RO] * dS, rp = S[RO] * p2;
+        baM -= fU * sv + rd * bd;
+        bUh[bn] -= f1 * c * sv + 2 * Ubn * (be + bd);
+        bS[RO] += dS * (dS * be + p2 * bd);
+        baS += 2 * rd * be + (rp + rd) * bd;
+        bS[vn] += fU * sv - 2 * rd * be - rp * bd;
+      };
+      star(R, bR, tR, kR, aR, kR * (central ? aR - aR1 : aR), dR, idR, roR, ER, ptR, vBR, f1R, gR, v1R, v2R, b1R, b2R,
+           bv1R, bv2R, bb1R, bb2R, baR, broR, bER, bptR, bvBR);
+      star(L, bL, tL, kL, aL, kL * (central ? aL - aL1 : aL), dL, idL, roL, EL, ptL, vBL, f1L, gL, v1L, v2L, b1L, b2L,
+           bv1L, bv2L, bb1L, bb2L, baL, broL, bEL, bptL, bvBL);
     }
-    // aVS = |Uh[bn]| / sqrt(roS)
+    // roS = S[RO] (aS - vn) / (aS - aM)
+    const double nL = broL * idL, nR = broR * idR;
+    bL[RO] += dL * nL;
+    baL += (L[RO] - roL) * nL;
+    bL[vn] -= L[RO] * nL;
+    bR[RO] += dR * nR;
+    baR += (R[RO] - roR) * nR;
+    bR[vn] -= R[RO] * nR;
+    baM += roL * nL + roR * nR;
+    // pt = ptL + L[RO] (aL - vn) (aM - vn)
     {
-      const double sg = slope_abs(Uh[bn]);
-      const double irL = 1.0 / roL, irR = 1.0 / roR;
-      bUh[bn] += sg * (baVL * sroL * irL + baVR * sroR * irR);  // 1/sqrt(ro) = sqrt(ro)/ro
-      broL -= 0.5 * baVL * aVL * irL;
-      broR -= 0.5 * baVR * aVR * irR;
-    }
-    // roS = S[RO] (aS - S[vn]) / (aS - aM)
-    for (int side = 1; side >= 0; side--) {
-      const bool Ls = side == 0;
-      const double *S = Ls ? L : R;
-      double *bS = Ls ? bL : bR;
-      const double aS = Ls ? aL : aR;
-      const double roS = Ls ? roL : roR;
-      const double b = Ls ? broL : broR;
-      double &baS = Ls ? baL : baR;
-      const double bnum = b / (aS - aM);
-      const double bden = -bnum * roS;
-      bS[RO] += (aS - S[vn]) * bnum;
-      baS += S[RO] * bnum + bden;
-      bS[vn] -= S[RO] * bnum;
-      baM -= bden;
-    }
-    // pt = ptL + L[RO] (aL - L[vn]) (aM - L[vn])
-    {
+      const double c = aM - L[vn], bc1 = c * bpt, bc2 = L[RO] * dL * bpt;
       bptL += bpt;
-      const double c1 = L[RO] * (aL - L[vn]), c2 = aM - L[vn];
-      const double bc1 = c2 * bpt, bc2 = c1 * bpt;
-      bL[RO] += (aL - L[vn]) * bc1;
+      bL[RO] += dL * bc1;
       baL += L[RO] * bc1;
       bL[vn] -= L[RO] * bc1 + bc2;
       baM += bc2;
     }
     // aM = Uh[mn] / Uh[RO]
-    {
-      const double iro = 1.0 / Uh[RO];
-      bUh[mn] += baM * iro;
-      bUh[RO] -= baM * aM * iro;
-    }
-    // Uh[m] = iw (aR XR[m] - aL XL[m] - FR[m] + FL[m])
+    bUh[mn] += baM * iro;
+    bUh[RO] -= baM * aM * iro;
+    // Uh = iw (aR UR - aL UL - FR + FL), iw = 1 / (aR - aL)
+    double g = 0;
     for (int m = 0; m < 8; m++) {
-      if (m == 3) continue;
-      const double XR = m < 3 ? UR[m] : R[m], XL = m < 3 ? UL[m] : L[m];
-      biw += (aR * XR - aL * XL - FR[m] + FL[m]) * bUh[m];
-      const double bN = iw * bUh[m];
-      baR += XR * bN;
-      baL -= XL * bN;
-      if (m < 3) {
-        bUR[m] += aR * bN;
-        bUL[m] -= aL * bN;
+      if (m == EN) continue;
+      const double b = iw * bUh[m];
+      g += Uh[m] * b;
+      if (m == bn) {
+        bR[bn] += aR * b;
+        bL[bn] -= aL * b;
+        baR += R[bn] * b;
+        baL -= L[bn] * b;
       } else {
-        bR[m] += aR * bN;
-        bL[m] -= aL * bN;
+        tL[m] += b;
+        tR[m] -= b;
       }
-      bFR[m] -= bN;
-      bFL[m] += bN;
     }
-    // iw = 1 / (aR - aL)
-    {
-      const double bw = -iw * iw * biw;
-      baR += bw;
-      baL -= bw;
+    baL += g - (L[RO] * (L[0] * tL[0] + L[1] * tL[1] + L[2] * tL[2]) + EL * tL[EN] + L[RO] * tL[RO] +
+                L[bt1] * tL[bt1] + L[bt2] * tL[bt2]);
+    baR -= g + (R[RO] * (R[0] * tR[0] + R[1] * tR[1] + R[2] * tR[2]) + ER * tR[EN] + R[RO] * tR[RO] +
+                R[bt1] * tR[bt1] + R[bt2] * tR[bt2]);
     }
   }
   // fan speeds: aL = min(vnL, vnR) - sa, aR = max(vnL, vnR) + sa, sa = sqrt(max(afL, afR))
-  {
-    if (L[vn] < R[vn]) bL[vn] += baL;
-    else bR[vn] += baL;
-    if (L[vn] > R[vn]) bL[vn] += baR;
-    else bR[vn] += baR;
-    const double bsa = baR - baL;
-    const double bm = bsa / (2 * sa);
-    double bafL = 0, bafR = 0;
-    if (afL > afR) bafL = bm;
-    else bafR = bm;
-    hlld_side_vjp<D>(L, bUL, bFL, bafL, bptL, bvBL, bL);
-    hlld_side_vjp<D>(R, bUR, bFR, bafR, bptR, bvBR, bR);
-  }
+  if (L[vn] < R[vn]) bL[vn] += baL;
+  else bR[vn] += baL;
+  if (L[vn] > R[vn]) bL[vn] += baR;
+  else bR[vn] += baR;
+  const double bm = (baR - baL) * (0.5 * rinv(sa));
+  side_vjp<D>(L, tL, eL, EL, ptL, vBL, afL, afL > afR ? bm : 0.0, bptL, bvBL, bEL, bL);
+  side_vjp<D>(R, tR, eR, ER, ptR, vBR, afR, afL > afR ? 0.0 : bm, bptR, bvBR, bER, bR);
 }
+
+#undef OMHD_STAR_ENERGY
+#undef OMHD_CONTRACT
 
 }  // namespace adj
 }  // namespace omhd

@@ -50,7 +50,6 @@
 namespace omhd {
 namespace {
 
-using adj::NV;
 
 struct Geo {
   long long plane, zstride;
@@ -377,9 +376,13 @@ __device__ __forceinline__ void face_vjp(const Geo &g, const double *__restrict_
 }
 
 // one thread per cell c along DIR: the face (c, c+1), or the high wall face.
-// MIR = false: axis DIR is periodic (only interior/periodic faces).
+// MIR = false: axis DIR is periodic (only interior/periodic faces).  Bound by
+// the issue of f64 arithmetic (about 2000 instructions a wavefront, 54% busy) and
+// near its 36 planes of traffic: 114 to 131 us on 192x96x80 cells against 88 at
+// the rate of a copy.  Two wavefronts per SIMD are asked for: a lone one
+// cannot cover its own latencies, and the walls' form is two registers over.
 template <int DIR, int LIM, bool MIR>
-__global__ __launch_bounds__(128) void k_adj_face(const Geo g, const double *__restrict__ w,
+__global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2, 8))) void k_adj_face(const Geo g, const double *__restrict__ w,
                                                   const double *__restrict__ M, double mscale, double mpsi, double ch,
                                                   double *__restrict__ AL, double *__restrict__ AR) {
   int i, j, k;
@@ -400,7 +403,7 @@ __global__ __launch_bounds__(128) void k_adj_face(const Geo g, const double *__r
 
 // walls only: one thread per cell of the plane c = 0, the low wall face
 template <int DIR, int LIM>
-__global__ __launch_bounds__(128) void k_adj_face_lo(const Geo g, const double *__restrict__ w,
+__global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2, 8))) void k_adj_face_lo(const Geo g, const double *__restrict__ w,
                                                      const double *__restrict__ M, double mscale, double mpsi,
                                                      double ch, double *__restrict__ AL, double *__restrict__ AR) {
   const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
