@@ -141,11 +141,10 @@ OMHD_HD void lim_coef(int type, double wm, double w0, double wp, double cR[3], d
     kAR = kAL = kA;
     kBR = kBL = kB;
   } else if (type == 3) {
-    if (!(gA * gB <= 0)) {
-      const double S = gA + gB, iS2 = 1.0 / (S * S);
-      kAR = kAL = gB * gB * iS2;
-      kBR = kBL = gA * gA * iS2;
-    }
+    // by a select, as below
+    const double S = gA + gB, iS2 = 1.0 / (S * S);
+    kAR = kAL = gA * gB <= 0 ? 0.0 : gB * gB * iS2;
+    kBR = kBL = gA * gB <= 0 ? 0.0 : gA * gA * iS2;
   } else if (type == 4) {
     const double f1 = 1.0 / 6.0;
     const double s = csign(0.5, gA) + csign(0.5, gB);
@@ -153,20 +152,13 @@ OMHD_HD void lim_coef(int type, double wm, double w0, double wp, double cR[3], d
     const double mA = (aA < aB) ? slope_abs(gA) : 0.0, mB = (aA < aB) ? 0.0 : slope_abs(gB);
     const double m = tmin(aA, aB);
     const double c1 = f1 * (2 * gA + gB), c2 = f1 * (gA + 2 * gB);
-    if (m < tabs(c1)) {
-      kAR = s * mA;
-      kBR = s * mB;
-    } else {
-      kAR = s * slope_abs(c1) * 2 * f1;
-      kBR = s * slope_abs(c1) * f1;
-    }
-    if (m < tabs(c2)) {
-      kAL = s * mA;
-      kBL = s * mB;
-    } else {
-      kAL = s * slope_abs(c2) * f1;
-      kBL = s * slope_abs(c2) * 2 * f1;
-    }
+    // by selects: branches here took a kernel with 81 of them out of its registers
+    const bool i1 = m < tabs(c1), i2 = m < tabs(c2);
+    const double u1 = s * slope_abs(c1) * f1, u2 = s * slope_abs(c2) * f1;
+    kAR = i1 ? s * mA : 2 * u1;
+    kBR = i1 ? s * mB : u1;
+    kAL = i2 ? s * mA : u2;
+    kBL = i2 ? s * mB : 2 * u2;
   }
   // gA = w0 - wm, gB = wp - w0
   cR[0] = -kAR;

@@ -51,35 +51,48 @@ namespace omhd {
 namespace {
 
 
+// n / d for a d known to the host, 0 <= n < 2^32 (Granlund and Montgomery 1994:
+// a multiplication by the rounded-up reciprocal): 4 instructions, on the scalar
+// unit where n is uniform, against about 20 of a 32-bit division
+struct Div {
+  unsigned d, mul, s1, s2;
+};
+Div div_by(unsigned d) {
+  unsigned l = 0;
+  while (l < 32 && (1ull << l) < d) l++;
+  return Div{d, (unsigned)((((1ull << l) - d) << 32) / d + 1), l < 1 ? l : 1, l < 1 ? 0 : l - 1};
+}
+__device__ __forceinline__ unsigned quotient(unsigned n, const Div &v) {
+  const unsigned t = __umulhi(v.mul, n);
+  return (t + ((n - t) >> v.s1)) >> v.s2;
+}
+
+// cell counts and numbers are 32-bit: the adjoint's nine states of nine planes
+// (omhd_adjoint_create) pass the card's memory before 2^29 cells
 struct Geo {
+  // the step's state arrays: slot planes, rows of u_pitch doubles
+  long long u_plane, u_zstride;
+  // the adjoint's own arrays (w, AL, AR, lam, lam*): element m * plane +
+  // k * zstride + j * pitch + i, the nine slots of a row one after the other, so
+  // that a face's 36 streams lie in a few pages (192x96x80 cells: the face
+  // kernels 126, 112 and 104 us, 129, 120 and 111 with slot planes; the gather
+  // 355 and 351)
   long long plane, zstride;
-  int pitch, nx, ny, nz, nd;
+  int u_pitch, pitch, nx, ny, nz, nd;
+  Div by_nx, by_ny, by_nty;  // nty: row tiles along y (cell_of_tiled)
   int bc[3];               // OMHD_BC_* per axis
   unsigned slo[3], shi[3]; // slots negated in the low / high mirror ghosts
   const double *eta;       // resistive: 3 face arrays of (nx+2)*(ny+2), or null
   double dx;
 };
 
-// cell number t as its place i on row r (of ny * nz, fewer than 2^32): by a
-// 32-bit division where the grid allows (a 64-bit one is more instructions
-// than the smaller kernels here have)
-__device__ __forceinline__ void row_of(const Geo &g, unsigned long long t, int &i, unsigned &r) {
-  if ((unsigned long long)g.nx * g.ny * g.nz <= 0xffffffffull) {
-    r = (unsigned)t / (unsigned)g.nx;
-    i = (int)((unsigned)t - r * (unsigned)g.nx);
-  } else {
-    r = (unsigned)(t / (unsigned)g.nx);
-    i = (int)(t - (unsigned long long)r * (unsigned)g.nx);
-  }
-}
-
 __device__ __forceinline__ bool cell_of(const Geo &g, int &i, int &j, int &k) {
-  const unsigned long long t = (unsigned long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (unsigned long long)g.nx * g.ny * g.nz) return false;
-  unsigned r;
-  row_of(g, t, i, r);
-  k = (int)(r / (unsigned)g.ny);
-  j = (int)(r - (unsigned)k * (unsigned)g.ny);
+  const unsigned t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= (unsigned)g.nx * g.ny * g.nz) return false;
+  const unsigned r = quotient(t, g.by_nx), q = quotient(r, g.by_ny);
+  i = (int)(t - r * g.nx);
+  j = (int)(r - q * g.ny);
+  k = (int)q;
   return true;
 }
 
@@ -93,12 +106,12 @@ __device__ __forceinline__ bool cell_of(const Geo &g, int &i, int &j, int &k) {
 __device__ __forceinline__ bool cell_of_tiled(const Geo &g, int &i, int &j, int &k) {
   const unsigned nb = gridDim.x, b = blockIdx.x;
   const unsigned L = (nb % 8u == 0u) ? (b % 8u) * (nb / 8u) + b / 8u : b;
-  const unsigned long long t = (unsigned long long)L * blockDim.x + threadIdx.x;
-  if (t >= (unsigned long long)g.nx * g.ny * g.nz) return false;
-  unsigned q;  // row ordinal in visiting order, < ny * nz
-  row_of(g, t, i, q);
+  const unsigned t = L * blockDim.x + threadIdx.x;
+  if (t >= (unsigned)g.nx * g.ny * g.nz) return false;
+  const unsigned q = quotient(t, g.by_nx);  // row ordinal in visiting order, < ny * nz
+  i = (int)(t - q * g.nx);
   const unsigned TY = min(16, g.ny & -g.ny), TZ = min(8, g.nz & -g.nz);  // powers of two
-  const unsigned in = q & (TY * TZ - 1), T = q / (TY * TZ), nty = (unsigned)g.ny / TY, tz = T / nty;
+  const unsigned in = q & (TY * TZ - 1), T = q / (TY * TZ), nty = (unsigned)g.ny / TY, tz = quotient(T, g.by_nty);
   j = (int)((T - tz * nty) * TY + (in & (TY - 1)));
   k = (int)(tz * TZ + in / TY);
   return true;
@@ -167,9 +180,10 @@ __global__ __launch_bounds__(256) void k_adj_prim(const Geo g, const double *__r
   int i, j, k;
   if (!cell_of(g, i, j, k)) return;
   const long long o = (long long)k * g.zstride + (long long)j * g.pitch + i;
+  const long long ou = (long long)k * g.u_zstride + (long long)j * g.u_pitch + i;
   double u[NV], p[NV];
 #pragma unroll
-  for (int m = 0; m < NV; m++) u[m] = U[m * g.plane + o];
+  for (int m = 0; m < NV; m++) u[m] = U[m * g.u_plane + ou];
   u[8] = psi_f * u[8];
   adj::prim_fwd<double>(u, p);
 #pragma unroll
@@ -414,16 +428,12 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2, 8))) voi
   face_vjp<DIR, LIM>(g, w, M, mscale, mpsi, ch, AL, AR, i, j, k, 2);
 }
 
-// the resistive flux's reverse at every face along DIR, first half: one
-// thread per cell c (the face (c, c+1), or the high wall face), plus the low
-// wall face for c = 0 at a wall; bF is rebuilt from mu as the face kernels
-// build it.  rf: the face arrays of all three axes.
+// the resistive flux's reverse, first half, at cell (i, j, k)'s faces along DIR:
+// the face (c, c+1), or the high wall face, plus the low wall face for c = 0 at
+// a wall; bF is rebuilt from mu as the face kernels build it
 template <int DIR>
-__global__ __launch_bounds__(256) void k_adj_res(const Geo g, const double *__restrict__ w,
-                                                 const double *__restrict__ M, double mscale, double mpsi,
-                                                 double *__restrict__ rf) {
-  int i, j, k;
-  if (!cell_of(g, i, j, k)) return;
+__device__ __forceinline__ void res_faces(const Geo &g, const double *__restrict__ w, const double *__restrict__ M,
+                                          double mscale, double mpsi, double *__restrict__ rf, int i, int j, int k) {
   const int c = DIR == 0 ? i : (DIR == 1 ? j : k);
   const int n = DIR == 0 ? g.nx : (DIR == 1 ? g.ny : g.nz);
   const bool wall = g.bc[DIR] != OMHD_BC_PERIODIC;
@@ -441,6 +451,19 @@ __global__ __launch_bounds__(256) void k_adj_res(const Geo g, const double *__re
     if (kind == 2) resistive_face<DIR>(g, w, i - (DIR == 0), j - (DIR == 1), k - (DIR == 2), bF, F);
     else resistive_face<DIR>(g, w, i, j, k, bF, F);
   }
+}
+// one thread per cell, all three axes: they read the same B and mu planes (22
+// planes in and out together, 33 one axis at a time).  rf: the face arrays.
+// 127 us on 192x96x80 cells at two wavefronts per SIMD (202 registers; three or
+// four spill: 157 and 290 us), 142 in three launches.
+__global__ __launch_bounds__(256) void k_adj_res(const Geo g, const double *__restrict__ w,
+                                                 const double *__restrict__ M, double mscale, double mpsi,
+                                                 double *__restrict__ rf) {
+  int i, j, k;
+  if (!cell_of_tiled(g, i, j, k)) return;
+  res_faces<0>(g, w, M, mscale, mpsi, rf, i, j, k);
+  res_faces<1>(g, w, M, mscale, mpsi, rf, i, j, k);
+  res_faces<2>(g, w, M, mscale, mpsi, rf, i, j, k);
 }
 
 // res_gather for a cell one or more cells from every wall: each role's
@@ -506,9 +529,9 @@ __global__ __launch_bounds__(256) void k_adj_res_gather(const Geo g, const doubl
     res_gather<1>(g, rf + fbase_of(g, 1), i, j, k, b);
     res_gather<2>(g, rf + fbase_of(g, 2), i, j, k, b);
   }
-  const long long o = (long long)k * g.zstride + (long long)j * g.pitch + i;
+  const long long o = (long long)k * g.u_zstride + (long long)j * g.u_pitch + i;
 #pragma unroll
-  for (int m = 0; m < 3; m++) R[m * g.plane + o] = b[m];
+  for (int m = 0; m < 3; m++) R[m * g.u_plane + o] = b[m];
 }
 
 // the eta adjoints: one thread per entry (DIR, i+1, j+1) of geta, the face
@@ -610,7 +633,7 @@ __global__ __launch_bounds__(256) void k_adj_gather(const Geo g, const double *_
   }
   if (R) {
 #pragma unroll
-    for (int m = 5; m < 8; m++) b[m] += R[(m - 5) * g.plane + o0];
+    for (int m = 5; m < 8; m++) b[m] += R[(m - 5) * g.u_plane + (ND == 3 ? k * g.u_zstride + (long long)j * g.u_pitch + i : o0)];
   }
   double nu[NV];
 #pragma unroll
@@ -637,7 +660,6 @@ __global__ void k_lam_copy(double *__restrict__ dst, const double *__restrict__ 
 }
 
 typedef void (*face_fn)(const Geo, const double *, const double *, double, double, double, double *, double *);
-typedef void (*res_fn)(const Geo, const double *, const double *, double, double, double *);
 typedef void (*gather_fn)(const Geo, const double *, const double *, const double *, long long, const double *,
                           const Combine);
 
@@ -665,8 +687,6 @@ face_fn face_kernel(int dir, int lo, bool mir, int lim) {
   if (dir == 1) return face_kernel<1>(lo, mir, lim);
   return face_kernel<2>(lo, mir, lim);
 }
-
-res_fn res_kernel(int dir) { return dir == 0 ? k_adj_res<0> : (dir == 1 ? k_adj_res<1> : k_adj_res<2>); }
 
 template <int ND, bool MIR>
 gather_fn gather_kernel(int lim) {
@@ -712,13 +732,19 @@ struct omhd_adjoint {
 
 static Geo geo_of(const omhd_handle *h) {
   Geo g;
-  g.plane = h->plane;
-  g.zstride = h->zstride;
-  g.pitch = h->pitch;
+  g.nd = h->nd;
+  g.u_plane = h->plane;
+  g.u_zstride = h->zstride;
+  g.u_pitch = h->pitch;
+  g.plane = h->pitch;
+  g.zstride = NV * h->zstride;
+  g.pitch = NV * h->pitch;
   g.nx = h->cfg.nx;
   g.ny = h->cfg.ny;
   g.nz = h->cfg.nz;
-  g.nd = h->nd;
+  g.by_nx = div_by(g.nx);
+  g.by_ny = div_by(g.ny);
+  g.by_nty = div_by(g.ny / std::min(16, g.ny & -g.ny));
   for (int a = 0; a < 3; a++) {
     g.bc[a] = h->faces.bc[a];
     g.slo[a] = h->faces.slo[a];
@@ -820,12 +846,10 @@ static int vjp_launch(omhd_adjoint *a, const double *W, double psi_f, const doub
                          g, a->w(), M, mscale, mpsi, ch, a->AL(dir), a->AR(dir));
       OMHD_HIP(hipGetLastError());
     }
-    if (res) {
-      hipLaunchKernelGGL(res_kernel(dir), dim3(g256), dim3(256), 0, h->stream, g, a->w(), M, mscale, mpsi, a->rf);
-      OMHD_HIP(hipGetLastError());
-    }
   }
   if (res) {
+    k_adj_res<<<g256, 256, 0, h->stream>>>(g, a->w(), M, mscale, mpsi, a->rf);
+    OMHD_HIP(hipGetLastError());
     k_adj_res_gather<<<g256, 256, 0, h->stream>>>(g, a->rf, a->R);
     OMHD_HIP(hipGetLastError());
     const long long ne = 3LL * (g.nx + 2) * (g.ny + 2);
