@@ -841,13 +841,14 @@ __global__ void k_solo_dt(SoloDev *s, unsigned long long *red, double cfl, doubl
 
 // CFL speed of the resident state (set_dt.f90:21-45), used once after upload.
 // Bound by memory (72 B per cell) on large grids and by the atomics, all to one
-// address, on small ones: the uploads of 48 members of 64^2 to 512^2, 1000^2
-// and 4096^2 grids together 12.0 us a call on average, 16 to 17 with 64-bit
-// divisions per cell and an atomic per wavefront; Harris 512x256x256 0.41 ms
-// either way (5.9 TB/s).
-template <int ND>
-__global__ __launch_bounds__(256) void k_cfl(const double *__restrict__ s, long long plane, long long zstride, int pitch,
-                                             int nx, int ny, int nz, unsigned long long *vmax_bits, int *err) {
+// address, on small ones: over the members of a 48-member ensemble (64^2 to
+// 512^2) 6.6 us a call, 16.6 with 64-bit divisions per cell and an atomic per
+// wavefront; Harris 512x256x256 0.41 ms either way (5.9 TB/s).  UP: the state is
+// brought in from a Fortran array on the way (10.1 us, 12.4 in two kernels).
+template <int ND, bool UP>
+__global__ __launch_bounds__(256) void k_cfl(double *__restrict__ s, const double *__restrict__ U, long long plane,
+                                             long long zstride, int pitch, int nx, int ny, int nz,
+                                             unsigned long long *vmax_bits, int *err) {
   __shared__ double wv[4];
   const int chunks = (nx + 63) / 64;
   const long long units = (long long)chunks * ny * nz;
@@ -859,10 +860,16 @@ __global__ __launch_bounds__(256) void k_cfl(const double *__restrict__ s, long 
     const int k = (int)(r / ny), j = (int)(r - (long long)k * ny);
     const int i = (int)(q - r * chunks) * 64 + threadIdx.x % 64;
     if (i < nx) {
-      const double *__restrict__ cell = s + k * zstride + (long long)j * pitch + i;
+      double *__restrict__ cell = s + k * zstride + (long long)j * pitch + i;
+      // UP: the interior of the Fortran array U(ix,jx[,kx],9)
+      const long long ix = nx + 2, jx = ny + 2, nf = ix * jx * (ND == 3 ? nz + 2 : 1);
+      const double *__restrict__ in = U + (((ND == 3 ? k + 1 : 0) * jx + (j + 1)) * ix + (i + 1));
       double u[NV], w[NV];
 #pragma unroll
-      for (int m = 0; m < NV; m++) u[m] = cell[m * plane];
+      for (int m = 0; m < NV; m++) {
+        u[m] = UP ? in[m * nf] : cell[m * plane];
+        if (UP) cell[m * plane] = u[m];
+      }
       const bool moderate = cons_to_prim(u, w);
       const int kk = ND == 3 ? k + 2 : 0;
       if (!(w[3] > 0.0) || !(u[4] > 0.0))
@@ -909,19 +916,9 @@ __global__ void k_to_fortran(const double *__restrict__ s, long long plane, long
   }
 }
 
-__global__ void k_from_fortran(const double *__restrict__ U, double *__restrict__ s, long long plane, long long zstride,
-                               int pitch, int nx, int ny, int nz, int nd) {
-  const int ix = nx + 2, jx = ny + 2, kx = nd == 3 ? nz + 2 : 1;
-  const long long gid = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (gid >= (long long)nx * ny * nz) return;
-  const int i = (int)(gid % nx);
-  const long long r = gid / nx;
-  const int j = (int)(r % ny), k = (int)(r / ny);
-  const long long n = (long long)ix * jx * kx;
-  const long long fk = nd == 3 ? k + 1 : 0;
-  const long long f = (fk * jx + (j + 1)) * ix + (i + 1);
-#pragma unroll
-  for (int m = 0; m < NV; m++) s[m * plane + (long long)k * zstride + (long long)j * pitch + i] = U[m * n + f];
+__global__ void k_zero_member(int *err, unsigned long long *vmax_bits) {
+  if (threadIdx.x < 8) err[threadIdx.x] = 0;
+  if (threadIdx.x == 8) *vmax_bits = 0;
 }
 
 __global__ void k_zero_red(unsigned long long *red) {
@@ -1294,16 +1291,13 @@ static unsigned cfl_grid(int nx, int ny, int nz) {
   return (unsigned)std::min<size_t>(((size_t)((nx + 63) / 64) * ny * nz + 3) / 4, 2048);
 }
 
-static int cfl_pass(omhd_handle *h) {
+// U: the Fortran array the state comes from (device memory), or null
+static int cfl_pass(omhd_handle *h, const double *U = nullptr) {
   const omhd_config &c = h->cfg;
   k_zero_red<<<1, 64, 0, h->stream>>>(h->red);
-  const unsigned grid = cfl_grid(c.nx, c.ny, h->nd == 3 ? c.nz : 1);
-  if (h->nd == 3)
-    k_cfl<3><<<grid, 256, 0, h->stream>>>(h->U, h->plane, h->zstride, h->pitch, c.nx, c.ny, c.nz, h->red,
-                                          (int *)(h->red + 1));
-  else
-    k_cfl<2><<<grid, 256, 0, h->stream>>>(h->U, h->plane, h->zstride, h->pitch, c.nx, c.ny, c.nz, h->red,
-                                          (int *)(h->red + 1));
+  const auto k = h->nd == 3 ? (U ? k_cfl<3, true> : k_cfl<3, false>) : (U ? k_cfl<2, true> : k_cfl<2, false>);
+  k<<<cfl_grid(c.nx, c.ny, c.nz), 256, 0, h->stream>>>(h->U, U, h->plane, h->zstride, h->pitch, c.nx, c.ny, c.nz, h->red,
+                                                       (int *)(h->red + 1));
   OMHD_HIP(hipGetLastError());
   int err[4];
   double vm;
@@ -1315,14 +1309,10 @@ static int cfl_pass(omhd_handle *h) {
 
 extern "C" int omhd_upload(omhd_handle *h, const double *U) {
   if (!h || !U) return set_error(OMHD_ERR_ARG, "null argument");
-  const omhd_config &c = h->cfg;
   Staged a;
   if (int rc = a.init(U, 9 * nfortran(h), true, false, h->stream)) return rc;
-  k_from_fortran<<<(unsigned)((ncells(h) + 255) / 256), 256, 0, h->stream>>>(a.dev, h->U, h->plane, h->zstride,
-                                                                             h->pitch, c.nx, c.ny, c.nz, h->nd);
-  OMHD_HIP(hipGetLastError());
+  if (int rc = cfl_pass(h, a.dev)) return rc;
   a.release(h->stream);
-  if (int rc = cfl_pass(h)) return rc;
   h->have_state = true;
   return ok();
 }
@@ -1933,17 +1923,12 @@ extern "C" int omhd_batch_upload(omhd_batch *b, int32_t i, const double *U) {
   const size_t nf = (size_t)(p.nx + 2) * (p.ny + 2);
   Staged a;
   if (int rc = a.init(U, 9 * nf, true, false, b->stream)) return rc;
-  k_from_fortran<<<(unsigned)(((size_t)p.nx * p.ny + 255) / 256), 256, 0, b->stream>>>(a.dev, p.U, p.plane, p.zstride,
-                                                                                        p.pitch, p.nx, p.ny, 1, 2);
+  // the state and its first CFL speed (main.f90:40)
+  k_zero_member<<<1, 64, 0, b->stream>>>(b->err_d, b->vmax_d + i);
+  k_cfl<2, true><<<cfl_grid(p.nx, p.ny, 1), 256, 0, b->stream>>>(p.U, a.dev, p.plane, p.zstride, p.pitch, p.nx, p.ny, 1,
+                                                                 b->vmax_d + i, b->err_d);
   OMHD_HIP(hipGetLastError());
   a.release(b->stream);
-  // first CFL speed of this member (main.f90:40)
-  OMHD_HIP(hipMemsetAsync(b->err_d, 0, 8 * sizeof(int), b->stream));
-  OMHD_HIP(hipMemsetAsync(b->vmax_d + i, 0, sizeof(unsigned long long), b->stream));
-  k_cfl<2><<<cfl_grid(p.nx, p.ny, 1), 256, 0, b->stream>>>(p.U, p.plane, p.zstride, p.pitch,
-                                                                                  p.nx, p.ny, 1, b->vmax_d + i,
-                                                                                  b->err_d);
-  OMHD_HIP(hipGetLastError());
   unsigned long long v;
   OMHD_HIP(hipMemcpyAsync(&v, b->vmax_d + i, sizeof v, hipMemcpyDeviceToHost, b->stream));
   if (int rc = batch_check_err(b)) return rc;
