@@ -134,8 +134,8 @@ namespace {
 // What u2v and set_dt hand back besides arrays, without an allocation, a fill
 // and a copy per call (those and a second wait were 35 of the 50 us a call
 // took on 202^2 cells): `out`, two words of pinned host memory that the kernel
-// writes and the call reads after its one wait, and `red`, three device words
-// that every launch leaves zero.  CALL_SLOTS calls may be under way at once, in
+// writes and the call reads after its one wait, and `red`, two device words
+// that every call leaves zero.  CALL_SLOTS calls may be under way at once, in
 // any threads; a further one waits for a slot to be given back.
 constexpr int CALL_SLOTS = 64;
 struct CallSlot {
@@ -157,8 +157,8 @@ struct CallSlot {
       unsigned long long *d = nullptr;
       if (!p.out)
         OMHD_HIP(hipHostMalloc((void **)&p.out, 2 * CALL_SLOTS * sizeof *p.out, hipHostMallocMapped | hipHostMallocCoherent));
-      OMHD_HIP(hipMallocAsync((void **)&d, 3 * CALL_SLOTS * sizeof *d, s));
-      OMHD_HIP(hipMemsetAsync(d, 0, 3 * CALL_SLOTS * sizeof *d, s));
+      OMHD_HIP(hipMallocAsync((void **)&d, 2 * CALL_SLOTS * sizeof *d, s));
+      OMHD_HIP(hipMemsetAsync(d, 0, 2 * CALL_SLOTS * sizeof *d, s));
       OMHD_HIP(hipStreamSynchronize(s));
       p.red = d;
       for (int i = 0; i < CALL_SLOTS; i++) p.free_ids.push_back(i);
@@ -167,7 +167,7 @@ struct CallSlot {
     id = p.free_ids.back();
     p.free_ids.pop_back();
     out = p.out + 2 * id;
-    red = p.red + 3 * id;
+    red = p.red + 2 * id;
     out[0] = out[1] = 0;
     return OMHD_OK;
   }
@@ -375,8 +375,7 @@ __device__ __forceinline__ void group_reduce(double &v, int &f) {
 
 // ---------------------------------------------------------------------------
 // set_dt: per-cell fastest speed, one atomic per workgroup, max bits in red[0],
-// flags in red[1]; the workgroup that red[2] counts last hands them to out and
-// clears red for the next launch.  SPEED_GROUPS
+// flags in red[1].  SPEED_GROUPS
 // workgroups at most, each over many cells: the atomics and the reads before
 // them all go to one address, so their number is bounded, and 2048 workgroups
 // fill the chip.  Bound by memory (64 B per cell).  160x128x120 cells: 40 us,
@@ -385,7 +384,7 @@ __device__ __forceinline__ void group_reduce(double &v, int &f) {
 constexpr unsigned SPEED_GROUPS = 2048;
 template <int ND>
 __global__ __launch_bounds__(256) void k_speed(const double *__restrict__ U, const double *__restrict__ V, int ix, int jx, int kx,
-                        unsigned long long *red, unsigned long long *out) {
+                        unsigned long long *red) {
   const Box b = speed_box(ix, jx, kx);
   const size_t total = b.count(), n = (size_t)ix * jx * kx, step = (size_t)gridDim.x * blockDim.x;
   double vt = 0.0;
@@ -402,13 +401,15 @@ __global__ __launch_bounds__(256) void k_speed(const double *__restrict__ U, con
     if (f & 8) vt = __builtin_nan("");
     if (f) atomicOr(&red[1], 4ull);
     atomic_max_nonneg(&red[0], vt);
-    __threadfence();
-    if (atomicAdd(&red[2], 1ull) == gridDim.x - 1) {  // the last workgroup
-      __threadfence();
-      out[0] = atomicExch(&red[0], 0ull);
-      out[1] = atomicExch(&red[1], 0ull);
-      atomicExch(&red[2], 0ull);
-    }
+  }
+}
+// hands k_speed's result to the host and clears it for the next call.  (The
+// last workgroup doing this by a ticket needs a device-wide fence in each of
+// them: k_speed took 160 us instead of 40 on 160x128x120 cells.)
+__global__ void k_speed_out(unsigned long long *red, unsigned long long *out) {
+  if (threadIdx.x < 2) {
+    out[threadIdx.x] = red[threadIdx.x];
+    red[threadIdx.x] = 0;
   }
 }
 
@@ -852,9 +853,10 @@ extern "C" int omhd_set_dt(const double *U, const double *V, double *vmax, doubl
   if (int rc = slot.acquire(s)) return rc;
   const unsigned groups = std::min(nblocks(speed_box(ix, jx, kx).count()), SPEED_GROUPS);
   if (ndim == 3)
-    k_speed<3><<<groups, TPB, 0, s>>>(a.dev, b.dev, ix, jx, kx, slot.red, slot.out);
+    k_speed<3><<<groups, TPB, 0, s>>>(a.dev, b.dev, ix, jx, kx, slot.red);
   else
-    k_speed<2><<<groups, TPB, 0, s>>>(a.dev, b.dev, ix, jx, kx, slot.red, slot.out);
+    k_speed<2><<<groups, TPB, 0, s>>>(a.dev, b.dev, ix, jx, kx, slot.red);
+  k_speed_out<<<1, 64, 0, s>>>(slot.red, slot.out);
   OMHD_HIP(hipGetLastError());
   a.release(s);
   b.release(s);
