@@ -1100,7 +1100,8 @@ extern "C" int omhd_create(const omhd_config *cfg, omhd_handle **out) {
   } else {
     const long long slots = march_slots(), strips = (cfg->nx + STRIP - 1) / STRIP;
     const long long slices = cfg->ndim == 3 ? nz : 1;
-    // the resistive XY pass's LDS leaves room for 7 wavefronts per CU, not 8
+    // the resistive XY pass's LDS leaves room for 7 wavefronts per CU, not 8 (Harris
+    // 64^3, a stage pair: 202 us with 7, more than the 229 of 8-row chunks with 8)
     h->rows = default_rows([&](int r) { return strips * slices * ((cfg->ny + r - 1) / r); }, cfg->ny, cfg->ndim,
                            cfg->resistive ? slots / 8 * 7 : slots);
     h->rows_z = default_rows([&](int r) { return strips * cfg->ny * (long long)((nz + r - 1) / r); }, nz, 3, slots);
