@@ -199,11 +199,13 @@ __device__ __forceinline__ void limit(double wm, double w0, double wp, double &g
 // sweep direction; L, R are interface states in the slot convention above.
 //
 // `moderate` (uniform across the wavefront): both states come from moderate
-// cells (cons_to_prim; the limiters keep a face state between its cells).
-// Then all of the quotients and roots below are in the range of quot and
-// sqrt_core except where the flow makes an operand small by cancellation;
-// those are tested, and a wavefront that has one forms the same values with
-// `/` and sqrt, there and from there on.
+// cells (cons_to_prim), and a limiter keeps a face state between its cells but
+// for rounding: where MC or Koren take the whole difference, w0 - (w0 - wm) is
+// zero for a wm below half an ulp of w0, so the face's own density and pressure
+// are tested.  Then all of the quotients and roots below are in the range of
+// quot and sqrt_core except where the flow makes an operand small by
+// cancellation; those are tested, and a wavefront that has one forms the same
+// values with `/` and sqrt, there and from there on.
 //
 // What only the side of the contact that the flux is taken from needs (its
 // energies and the rest of its physical flux) is formed inside that side's
@@ -241,7 +243,12 @@ __device__ __forceinline__ void hlld(const double L[NV], const double R[NV], dou
   constexpr int vn = D, vt1 = (D + 1) % 3, vt2 = (D + 2) % 3;  // :62-70
   constexpr int bn = 5 + vn, bt1 = 5 + vt1, bt2 = 5 + vt2;
   constexpr int RO = 4, PR = 3, EN = 3;
-  bool slow = !moderate;
+  // a value is at least MOD_LO where its high word is (compared as integers: a
+  // negative value has a negative one)
+  const int lo = __double2hiint(MOD_LO);
+  const int mL0 = min(__double2hiint(L[RO]), __double2hiint(L[PR]));
+  const int mR0 = min(__double2hiint(R[RO]), __double2hiint(R[PR]));
+  bool slow = !moderate || any_lane(min(mL0, mR0) < lo);
 
   // fast speed^2 and total pressure of each side; q is 0 or >= 2^-260
   const double B2L = dot3(L + 5, L + 5), B2R = dot3(R + 5, R + 5);
@@ -291,8 +298,6 @@ __device__ __forceinline__ void hlld(const double L[NV], const double R[NV], dou
     double aVR = quot(__builtin_fabs(hb), sroR, recip(sroR));  // :437
     {
       // positive and not small: hro, aM - aL, aR - aM, L vn - aL, aR - R vn
-      // (high words compared as integers: a negative value has a negative one)
-      const int lo = __double2hiint(MOD_LO);
       const int m3 = min(min(__double2hiint(hro), __double2hiint(-eL)), __double2hiint(eR));
       const int m5 = min(min(m3, __double2hiint(-dL)), __double2hiint(dR));
       slow = slow || any_lane(fan && (m5 < lo || tiny(hmn) || tiny(hb)));
