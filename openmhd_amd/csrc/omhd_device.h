@@ -433,14 +433,15 @@ __device__ __forceinline__ void hlld(const double L[NV], const double R[NV], dou
     if (!fan) {
       // F(L) where aL >= 0, else F(R).  A NaN speed has aL >= 0, aR <= 0 and
       // the fan's tests all false; the reference's chain of tests then ends in
-      // the fan, and any NaN flux says the same
+      // the fan, whose flux is NaN (an infinite speed makes one edge NaN and
+      // leaves the other infinite)
       double S[8];
 #pragma unroll
       for (int m = 0; m < 8; m++) S[m] = aL >= 0 ? L[m] : R[m];
       side_flux<D>(S, dot3(S, S), dot3(S + 5, S + 5), dot3(S, S + 5), F);
       if (!(aL >= 0) && !(aR <= 0)) {
 #pragma unroll
-        for (int m = 0; m < 8; m++) F[m] = aR;
+        for (int m = 0; m < 8; m++) F[m] = __builtin_nan("");
       }
     }
   }

@@ -98,3 +98,24 @@ def test_step_with_vanishing_fields(oracle, nx, ny, lm, tt):
     O = U.copy(order="F")
     assert oracle.run(p, O, 12)[0] == 0
     assert same(G, O)
+
+
+@pytest.mark.parametrize("dir", (1, 2))
+def test_flux_of_infinite_states(oracle, dir):
+    """Infinite velocities and pressures: where an infinite fast speed takes the
+    fan's edge to NaN, so is the flux."""
+    from openmhd_amd import api
+
+    cases = [(v, p, w, q) for v in (1.0, np.inf, -np.inf) for p in (1.0, np.inf) for w in (1.0, np.inf, -np.inf)
+             for q in (1.0, np.inf)]
+    shape = (len(cases) + 2, 5) if dir == 1 else (5, len(cases) + 2)
+    VL, VR = states(4, shape, SCALES[:1]), states(5, shape, SCALES[:1])
+    for i, (v, p, w, q) in enumerate(cases):
+        at = (i + 1, slice(None)) if dir == 1 else (slice(None), i + 1)
+        VL[at + (dir - 1,)], VL[at + (3,)] = v, p
+        VR[at + (dir - 1,)], VR[at + (3,)] = w, q
+    F1, F2 = farr(*shape, 9), farr(*shape, 9)
+    with np.errstate(all="ignore"):
+        oracle.flux_solver(F2, VL, VR, 1.3, dir, 3)
+    api.flux_solver(F1, VL, VR, 1.3, *shape, dir, 3)
+    assert same(F1, F2)
