@@ -9,12 +9,12 @@
 #include <stdlib.h>
 
 #include <map>
-#include <condition_variable>
 #include <mutex>
 #include <vector>
 
 #include "omhd_device.h"
 #include "omhd_host.h"
+#include "omhd_slot.h"
 
 namespace omhd {
 
@@ -131,59 +131,6 @@ hipStream_t dropin_stream() {
 }
 
 namespace {
-// What u2v and set_dt hand back besides arrays, without an allocation, a fill
-// and a copy per call (those and a second wait were 35 of the 50 us a call
-// took on 202^2 cells): `out`, two words of pinned host memory that the kernel
-// writes and the call reads after its one wait, and `red`, two device words
-// that every call leaves zero.  CALL_SLOTS calls may be under way at once, in
-// any threads; a further one waits for a slot to be given back.
-constexpr int CALL_SLOTS = 64;
-struct CallSlot {
-  unsigned long long *out = nullptr, *red = nullptr;
-  int id = -1;
-  CallSlot() = default;
-  CallSlot(const CallSlot &) = delete;
-  CallSlot &operator=(const CallSlot &) = delete;
-  ~CallSlot() {
-    if (id < 0) return;
-    std::lock_guard<std::mutex> lock(pool().mu);
-    pool().free_ids.push_back(id);
-    pool().given_back.notify_one();
-  }
-  int acquire(hipStream_t s) {
-    Pool &p = pool();
-    std::unique_lock<std::mutex> lock(p.mu);
-    if (!p.red) {
-      unsigned long long *d = nullptr;
-      if (!p.out)
-        OMHD_HIP(hipHostMalloc((void **)&p.out, 2 * CALL_SLOTS * sizeof *p.out, hipHostMallocMapped | hipHostMallocCoherent));
-      OMHD_HIP(hipMallocAsync((void **)&d, 2 * CALL_SLOTS * sizeof *d, s));
-      OMHD_HIP(hipMemsetAsync(d, 0, 2 * CALL_SLOTS * sizeof *d, s));
-      OMHD_HIP(hipStreamSynchronize(s));
-      p.red = d;
-      for (int i = 0; i < CALL_SLOTS; i++) p.free_ids.push_back(i);
-    }
-    p.given_back.wait(lock, [&] { return !p.free_ids.empty(); });
-    id = p.free_ids.back();
-    p.free_ids.pop_back();
-    out = p.out + 2 * id;
-    red = p.red + 2 * id;
-    out[0] = out[1] = 0;
-    return OMHD_OK;
-  }
-
- private:
-  struct Pool {
-    std::mutex mu;
-    std::condition_variable given_back;
-    std::vector<int> free_ids;
-    unsigned long long *out = nullptr, *red = nullptr;
-  };
-  static Pool &pool() {
-    static Pool *p = new Pool;  // outlives every thread that may still hold a slot
-    return *p;
-  }
-};
 
 constexpr int TPB = 256;
 
@@ -701,6 +648,7 @@ extern "C" int omhd_u2v(const double *U, double *V, int32_t ix, int32_t jx, int3
   dU.release(s);
   dV.release(s);
   OMHD_HIP(hipStreamSynchronize(s));
+  slot.finished();
   if (slot.out[0]) {  // u2v.f90:34-38: report minloc of p
     double val;
     size_t c = plane_minloc(V + 3 * n, n, is_device_ptr(V), val);
@@ -856,11 +804,13 @@ extern "C" int omhd_set_dt(const double *U, const double *V, double *vmax, doubl
     k_speed<3><<<groups, TPB, 0, s>>>(a.dev, b.dev, ix, jx, kx, slot.red);
   else
     k_speed<2><<<groups, TPB, 0, s>>>(a.dev, b.dev, ix, jx, kx, slot.red);
+  OMHD_HIP(hipGetLastError());
   k_speed_out<<<1, 64, 0, s>>>(slot.red, slot.out);
   OMHD_HIP(hipGetLastError());
   a.release(s);
   b.release(s);
   OMHD_HIP(hipStreamSynchronize(s));
+  slot.finished();
   const unsigned long long h[2] = {slot.out[0], slot.out[1]};
   double vm;
   memcpy(&vm, &h[0], sizeof vm);
