@@ -161,3 +161,20 @@ def test_upload_in_device_dt_mode():
         assert bits_equal(e.download(i), Us), i
         assert bits_equal(e.times()[i], sum_in_order(dts)), i
     e.close()
+
+
+def test_autotune_times_the_default_height():
+    """Four members of 64 x 64: the library's own chunks have one or two rows
+    (a lone wavefront marches its rows one after the other), and taller ones
+    than 8 take several times as long.  The tuner times the height it found and
+    the low ones, so it cannot leave a small ensemble with tall chunks."""
+    from openmhd_amd import Ensemble
+
+    cfgs, states = members(n=4, seed=17, smin=64, smax=64)
+    e = Ensemble(cfgs)
+    for i, U in enumerate(states):
+        e.upload(i, U)
+    e.set_mode(device_dt=True)
+    rows, _ = e.autotune(20)
+    e.close()
+    assert 1 <= rows < 8
