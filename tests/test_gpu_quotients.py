@@ -119,3 +119,67 @@ def test_flux_of_infinite_states(oracle, dir):
         oracle.flux_solver(F2, VL, VR, 1.3, dir, 3)
     api.flux_solver(F1, VL, VR, 1.3, *shape, dir, 3)
     assert same(F1, F2)
+
+
+def conserved(W):
+    U = W.copy(order="F")
+    with np.errstate(all="ignore"):
+        for m in range(3):
+            U[..., m] = W[..., 4] * W[..., m]
+        U[..., 3] = W[..., 3] / (2.0 / 3.0) + 0.5 * (W[..., 4] * (W[..., :3] ** 2).sum(-1) + (W[..., 5:8] ** 2).sum(-1))
+    return U
+
+
+@pytest.mark.parametrize("scales", [SCALES] + [[s] for s in SCALES], ids=["mixed"] + [str(i) for i in range(len(SCALES))])
+def test_u2v_reports_every_bad_state(oracle, scales):
+    """u2v raises exactly where the oracle's does, with its code and cell."""
+    from openmhd_amd import OMHDError, api
+
+    shape = (131, 7)
+    U = conserved(states(3, shape, scales))
+    V1, V2 = farr(*shape, 4), farr(*shape, 4)
+    rc, bad = oracle.u2v(U, V2)
+    code, cell = 0, None
+    try:
+        api.u2v(U, V1, *shape)
+    except OMHDError as e:
+        code, cell = e.code, e.cell[:2]
+    assert code == rc and same(V1, V2)
+    assert rc == 0 or cell == (bad % shape[0] + 1, bad // shape[0] + 1)
+
+
+# states whose energy holds their pressure and whose jumps a step keeps positive
+MIXED, ALONE = [(0, 1, 4, 5, 6, 7, 8), (0, 2, 4, 5, 6, 7, 8)], (0, 1, 2, 3, 4, 5, 6, 7, 8, 10)
+
+
+@pytest.mark.parametrize("nz", (0, 5))
+@pytest.mark.parametrize("which", MIXED + [(i,) for i in ALONE],
+                         ids=["mixed low", "mixed high"] + [str(i) for i in ALONE])
+def test_speeds_of_a_run(oracle, which, nz):
+    """The CFL speed after an upload and after a step (first-order faces and a
+    tiny step, so that the states stay what they are): dt and ch of the first
+    two steps."""
+    from openmhd_amd import Solver
+
+    shape = (133, 9) + ((nz + 2,) if nz else ())
+    scales = [SCALES[i] for i in which]
+    W = states(6, shape, scales)
+    W[..., 8] = 0.0
+    ro, p = scales[0][:2]
+    b = 32 * 2.0 ** round(0.5 * np.log2(p))
+    W[5, 5] = 0.0  # gamma p = Bx^2 = B^2 in one column, the fastest: a zero inner root
+    W[5, 5, ..., 3], W[5, 5, ..., 4], W[5, 5, ..., 5] = 0.6 * b * b, ro, b
+    U = conserved(W)
+    V = farr(*shape, 4)
+    assert oracle.u2v(U, V)[0] == 0 and np.all(5 / 3 * V[5, 5, ..., 3] == b * b)
+    kw = dict(cfl=1e-9 if len(which) == 1 else 1e-40, lm_type=0, time_type=1)
+    dx = 4e-7 / kw["cfl"] * oracle.set_dt(U, V, 1.0, 1.0, ndim=3 if nz else 2)[1]
+    p = make_problem(*shape, dx=dx, **kw)
+    oracle.bc_u(U, p)
+    rc, dts, chs = oracle.run(p, U.copy(order="F"), 2)
+    assert rc == 0 and np.isfinite(chs).all()
+    s = Solver(shape[0] - 2, shape[1] - 2, dx, nz=nz, bc=("periodic",) * (3 if nz else 2), **kw)
+    s.upload(U)
+    got = s.step(2, trace=True)
+    s.close()
+    assert same(got[0], dts) and same(got[1], chs)
