@@ -365,7 +365,9 @@ OMHD_HD void hlld_fwd(const T L[NV], const T R[NV], double ch, T F[NV], int *bra
 #define OMHD_CONTRACT
 #endif
 
-// 1/x to an ulp
+// 1/x to an ulp, of any x: the fix-up gives what zeros, infinities and NaN give
+// and what over- and underflow, so unlike quot's its uses need no range.  (The
+// bits of 1.0 / x on 512 random values at each exponent, subnormals included.)
 OMHD_HD double rinv(double x) {
 #if defined(__HIP_DEVICE_COMPILE__)
   return __builtin_amdgcn_div_fixup(recip(x), x, 1.0);

@@ -74,9 +74,8 @@ struct Geo {
   long long u_plane, u_zstride;
   // the adjoint's own arrays (w, AL, AR, lam, lam*): element m * plane +
   // k * zstride + j * pitch + i, the nine slots of a row one after the other, so
-  // that a face's 36 streams lie in a few pages (192x96x80 cells: the face
-  // kernels 126, 112 and 104 us, 129, 120 and 111 with slot planes; the gather
-  // 355 and 351)
+  // that a face's 36 streams lie in a few pages (192x96x80 cells, the three face
+  // kernels together: 342 us, 360 with slot planes; the gather 355 and 351)
   long long plane, zstride;
   int u_pitch, pitch, nx, ny, nz, nd;
   Div by_nx, by_ny, by_nty;  // nty: row tiles along y (cell_of_tiled)
@@ -391,9 +390,9 @@ __device__ __forceinline__ void face_vjp(const Geo &g, const double *__restrict_
 
 // one thread per cell c along DIR: the face (c, c+1), or the high wall face.
 // MIR = false: axis DIR is periodic (only interior/periodic faces).  Bound by
-// the issue of f64 arithmetic (about 2000 instructions a wavefront, 54% busy) and
-// near its 36 planes of traffic: 114 to 131 us on 192x96x80 cells against 88 at
-// the rate of a copy.  Two wavefronts per SIMD are asked for: a lone one
+// the issue of f64 arithmetic (1310 to 1540 instructions a wavefront, 55 to 66%
+// busy) and near its 36 planes of traffic: 102 (x), 125 to 129 (y, the wall axis)
+// and 110 us (z) on 192x96x80 cells against 88 at the rate of a copy.  Two wavefronts per SIMD are asked for: a lone one
 // cannot cover its own latencies, and the walls' form is two registers over.
 template <int DIR, int LIM, bool MIR>
 __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2, 8))) void k_adj_face(const Geo g, const double *__restrict__ w,
@@ -454,7 +453,7 @@ __device__ __forceinline__ void res_faces(const Geo &g, const double *__restrict
 }
 // one thread per cell, all three axes: they read the same B and mu planes (22
 // planes in and out together, 33 one axis at a time).  rf: the face arrays.
-// 127 us on 192x96x80 cells at two wavefronts per SIMD (202 registers; three or
+// 126 us on 192x96x80 cells at two wavefronts per SIMD (202 registers; three or
 // four spill: 157 and 290 us), 142 in three launches.
 __global__ __launch_bounds__(256) void k_adj_res(const Geo g, const double *__restrict__ w,
                                                  const double *__restrict__ M, double mscale, double mpsi,
@@ -512,7 +511,7 @@ __device__ __forceinline__ void res_gather_inner(const Geo &g, const double *__r
 // second half: one thread per cell, the B adjoints from the faces of all
 // three axes, written to R (3 planes, slots bx, by, bz).  Bound by the loads (30
 // per cell, most of them from cache).  Only cells at a wall take the general
-// gather (82 us on 192x96x80 cells; 168 us when the ends of every periodic
+// gather (78 us on 192x96x80 cells; 168 us when the ends of every periodic
 // row took it too, and two of three wavefronts with them).
 __global__ __launch_bounds__(256) void k_adj_res_gather(const Geo g, const double *__restrict__ rf,
                                                         double *__restrict__ R) {

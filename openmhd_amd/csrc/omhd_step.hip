@@ -383,9 +383,9 @@ __device__ __forceinline__ double xo_term(const double a[4]) {
 // One tile: strip x chunk (x slice) of one grid.
 // The XY and 2D passes are bound by the vector unit's issue slots and by what
 // of a row's serial chain two wavefronts per SIMD leave uncovered; the Z pass
-// by HBM.  On KH 4096^2 (minmod) a row takes 1301 vector instructions in stage
-// 1 and 1453 in stage 2, two thirds of them the two flux evaluations, and the
-// vector unit issues in 80% and 75% of the cycles: 0.89 and 1.03 ms a stage.
+// by HBM.  On KH 4096^2 (minmod) a row takes 1300 vector instructions in stage
+// 1 and 1452 in stage 2, two thirds of them the two flux evaluations, and the
+// vector unit issues in 80% and 76% of the cycles: 0.89 and 1.04 ms a stage.
 // With a division for every quotient, 64-bit address arithmetic per access and
 // wall signs held in (spilled) scalar registers it was 1516 and 1687
 // instructions, 86% and 83% busy, 0.99 and 1.12 ms.  So what is not arithmetic
@@ -841,8 +841,8 @@ __global__ void k_solo_dt(SoloDev *s, unsigned long long *red, double cfl, doubl
 
 // CFL speed of the resident state (set_dt.f90:21-45), used once after upload.
 // Bound by memory (72 B per cell) on large grids and by the atomics, all to one
-// address, on small ones: over the members of a 48-member ensemble (64^2 to
-// 512^2) 6.6 us a call, 16.6 with 64-bit divisions per cell and an atomic per
+// address, on small ones: over the members of a 48-member ensemble (sides 65
+// to 765) 6.6 us a call, 16.6 with 64-bit divisions per cell and an atomic per
 // wavefront; Harris 512x256x256 0.41 ms either way (5.9 TB/s).  UP: the state is
 // brought in from a Fortran array on the way (10.1 us, 12.4 in two kernels).
 template <int ND, bool UP>
@@ -989,7 +989,10 @@ march_fn march_kernel(int pass, int res, int lim, int stage, int tt, bool gen = 
 // then takes 8.5 + 7 r, against 6 + 4.8 r for one that has the SIMD to itself,
 // and full rounds of `slots` chunks follow each other.  The 8.5 is what a
 // chunk pays before its first updated row (one load latency and two flux
-// evaluations).  3D passes scale alike, so the same line serves.
+// evaluations).  The 3D passes take the same line, for want of one of their own:
+// over eight grids of 48x32x20 to 512x256x256, ideal and resistive, the heights
+// it picks take 0.90 to 1.03 times the best single height for both passes (of
+// thirteen, 1 to 40 rows).
 double march_cost(long long tiles, int r, long long slots) {
   const long long full = tiles / slots, rest = tiles % slots;
   const double shared = 8.5 + 7.0 * r, alone = 6.0 + 4.8 * r;
@@ -1116,7 +1119,7 @@ extern "C" int omhd_create(const omhd_config *cfg, omhd_handle **out) {
     const long long slots = march_slots(), strips = (cfg->nx + STRIP - 1) / STRIP;
     const long long slices = cfg->ndim == 3 ? nz : 1;
     // the resistive XY pass's LDS leaves room for 7 wavefronts per CU, not 8 (Harris
-    // 64^3, a stage pair: 202 us with 7, 229 in 8-row chunks, more than that with 8)
+    // 64^3: 182 us a step, 201 in the best single height, 8 rows)
     h->rows = default_rows([&](int r) { return strips * slices * ((cfg->ny + r - 1) / r); }, cfg->ny, cfg->ndim,
                            cfg->resistive ? slots / 8 * 7 : slots);
     h->rows_z = default_rows([&](int r) { return strips * cfg->ny * (long long)((nz + r - 1) / r); }, nz, 3, slots);

@@ -1,6 +1,6 @@
 #!/bin/bash
 # The CPU test suite against AddressSanitizer + UndefinedBehaviorSanitizer
-# builds of the oracle (oracle/_san/liboracle.so) and of the native adjoint
+# builds of the oracle (oracle/_san/liboracle.so) and of the native
 # checkers (tests/native/_san/*.so).  Python itself is not instrumented, so the
 # sanitizer runtimes are preloaded; leak checking is off (the interpreter keeps
 # its allocations to the end).  Any report fails the run.
@@ -17,6 +17,6 @@ export OMHD_SANITIZED=1
 if [ $# -eq 0 ]; then
   set -- tests/test_oracle_golden.py tests/test_oracle_resistive3d.py tests/test_adjoint_cpu.py tests/test_flopcount.py \
     tests/test_brio_wu.py tests/test_recon2d.py tests/test_symmetry.py tests/test_invariants.py tests/test_snapshot.py \
-    tests/test_diagnostics.py -m "not gpu"
+    tests/test_diagnostics.py tests/test_call_slots.py -m "not gpu"
 fi
 exec python3 -m pytest -q -p no:cacheprovider "$@"
